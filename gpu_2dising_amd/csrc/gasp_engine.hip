@@ -19,6 +19,7 @@
 #include "gasp_internal.h"
 #include "gasp_kernels.h"
 #include "gasp_sliced.h"
+#include "gasp_window.h"
 
 using namespace gasp;
 
@@ -317,14 +318,18 @@ static size_t sliced_lds_bytes(int N) { return (size_t)kSlLat + (size_t)kSlEntry
 
 // Shapes picked by gasp_autotune, keyed by (method, L, ngrids); used when no
 // explicit gasp_set_tuning override is active.
-static std::map<std::tuple<int, int, int>, std::pair<int, int>> g_tuned;
+struct TunedShape {
+    int S, W;
+    bool window;  // the automatic sweep_window was faster than (S, W)
+};
+static std::map<std::tuple<int, int, int>, TunedShape> g_tuned;
 
 static void choose_tuning(int method, int L, int R, int *S_out, int *W_out) {
     if (g_tune_slots <= 0 && g_tune_waves <= 0) {
         auto it = g_tuned.find(std::make_tuple(method, L, R));
         if (it != g_tuned.end()) {
-            *S_out = it->second.first;
-            *W_out = it->second.second;
+            *S_out = it->second.S;
+            *W_out = it->second.W;
             return;
         }
     }
@@ -410,8 +415,8 @@ static void choose_sliced(int L, int R, int *S_out, int *W_out) {
     if (g_tune_slots <= 0 && g_tune_waves <= 0) {
         auto it = g_tuned.find(std::make_tuple(3, L, R));
         if (it != g_tuned.end()) {
-            *S_out = it->second.first;
-            *W_out = it->second.second;
+            *S_out = it->second.S;
+            *W_out = it->second.W;
             return;
         }
     }
@@ -564,6 +569,27 @@ static SweepFn sweep_fn(int method, int rng, int S, int W, bool pow2, int varian
                     : pick_sweep2<LAT_HBM, RNG_DRAWS>(S, pow2, variant);
 }
 
+// One replica per workgroup of `waves` waves (gasp_window.h).
+template <int RNG, bool P2, int MODE, int IO>
+static SweepFn pick_window(int waves) {
+    switch (waves) {
+        case 1: return sweep_window<RNG, 1, P2, MODE, IO>;
+        case 2: return sweep_window<RNG, 2, P2, MODE, IO>;
+        case 4: return sweep_window<RNG, 4, P2, MODE, IO>;
+        case 8: return sweep_window<RNG, 8, P2, MODE, IO>;
+        default: return nullptr;
+    }
+}
+template <int RNG, int IO>
+static SweepFn window_fn2(int waves, int mode, bool pow2) {
+    if (mode == WIN_TABLE) return pow2 ? pick_window<RNG, true, WIN_TABLE, IO>(waves) : pick_window<RNG, false, WIN_TABLE, IO>(waves);
+    return pow2 ? pick_window<RNG, true, WIN_PACKED, IO>(waves) : pick_window<RNG, false, WIN_PACKED, IO>(waves);
+}
+static SweepFn window_fn(int rng, int waves, int mode, bool pow2, int io) {
+    if (io == WIN_INT32) return rng == 0 ? window_fn2<RNG_PHILOX, WIN_INT32>(waves, mode, pow2) : nullptr;
+    return rng == 0 ? window_fn2<RNG_PHILOX, WIN_BITS>(waves, mode, pow2) : window_fn2<RNG_DRAWS, WIN_BITS>(waves, mode, pow2);
+}
+
 static bool is_pow2(int L) { return L > 0 && (L & (L - 1)) == 0; }
 static int ilog2(int L) {
     int g = 0;
@@ -582,7 +608,80 @@ struct LaunchShape {
     int ncu = 256;
     size_t lds = 0, lat_bytes = 0;
     bool sliced = false;  // method 3: sweep_sliced, S = waves per workgroup, W = word split (1: 64, 2: 32)
+    int win = 0;          // waves per replica of sweep_window (0: another kernel)
+    int wmode = 0;        // ... its MODE
 };
+
+// LDS of a sweep_window workgroup: a dword per site, or (M > 0) the bits and M keys.
+static size_t window_lds_bytes(int N, int M) {
+    return (size_t)kWinLat + (M > 0 ? (((size_t)N + 127) / 128) * 16 + 4 * (size_t)M : 4 * (size_t)N);
+}
+// Entries of its key table for per_cu workgroups on a CU: a power of two from
+// 1024, one per site up to what the LDS holds and 32768; 0: no room.
+static int window_table_entries(int N, size_t lds, int per_cu) {
+    const size_t per_wg = lds / (size_t)per_cu;
+    int M = 1024;
+    if (window_lds_bytes(N, M) > per_wg) return 0;
+    while (M < N && M < 32768 && window_lds_bytes(N, 2 * M) <= per_wg) M *= 2;
+    return M;
+}
+
+// Whether (method, L, R) runs on sweep_window, and its shape.  Its time grows
+// with the replicas as soon as the device is full, while the kernels that share
+// a workgroup between 8 to 64 replicas take as long for a few replicas as for
+// many, so it takes the smaller counts.  Method 2, 20 sweeps at L = 64: 256
+// replicas 0.21 ms against 2.11 on split words, 1024 0.37 against 2.14, 4096
+// 1.07 against 2.23, 8192 1.98 against 2.13, but 16384 3.70 against 3.20; 16384
+// at L = 48 2.07 against 2.10 and at L = 32 0.91 against 1.12; 8192 at L = 90
+// (10 sweeps) 2.13 against 2.15 and at L = 128 (5 sweeps) 2.38 against 2.41.
+// Method 1: 16384 at L = 64 (10 sweeps) 1.88 against 2.13, 65536 (5 sweeps)
+// 3.73 against 3.29, 16384 at L = 128 (2 sweeps) 2.10 against 1.68.  Method 0
+// is slower at every count: 16384 at L = 64 (10 sweeps) 1.90 against 3.01, 1024
+// at L = 256 (5 sweeps) 1.66 against 2.23.  An explicit shape, filter, staging
+// or table setting keeps the kernel that it is for.
+static void window_shape(int method, int L, int R, LaunchShape *sh) {
+    if (method > 2 || g_tune_slots > 0 || g_tune_waves > 0 || g_tune_filter == 1 || g_tune_filter == 2 ||
+        (g_tune_stage >= 1 && g_tune_stage <= 3) || g_tune_tables > 0)
+        return;
+    auto it = g_tuned.find(std::make_tuple(method, L, R));
+    if (it != g_tuned.end() && !it->second.window) return;
+    const long long ncu = sh->ncu;
+    if (!(method == 0 && L >= 32) && R > (L <= (method == 2 ? 48 : 64) ? 64 * ncu : 40 * ncu)) return;
+    DeviceInfo d = device_info();
+    const size_t lds = d.ok ? d.lds_block : 65536;
+    const int N = L * L;
+    const int want = std::max(1, (int)((R + ncu - 1) / ncu));  // workgroups a CU has to run
+    // A dword per site while two workgroups fit, or one where one is all there
+    // is: 256 replicas at L = 200 5% faster than with a table, 1024 (one
+    // resident workgroup against four) 16% slower.
+    int M = 0;
+    if (window_lds_bytes(N, 0) * (size_t)std::min(want, 2) > lds) {
+        M = window_table_entries(N, lds, std::min(want, 4));
+        if (M == 0) return;
+    }
+    const int res = std::min(want, (int)(lds / window_lds_bytes(N, M)));  // resident workgroups per CU
+    // Waves per replica: a window of 128 W attempts defers about 320 W / E of
+    // them (E entries), and a CU is full from about 16 waves on.  Measured
+    // fastest: 4 and 8 waves at L = 64 with 256 replicas (one workgroup per
+    // CU), 4 with 1024, 2 from 2048 on; 4 at L = 75 with 3001; 1 at L = 32 with
+    // 2048 and 2 with 256; 8 at L = 128 and 256 (sixteen never: 2.34 ms against
+    // 1.73 for 20 sweeps of 256 replicas at L = 256).
+    const int E = M > 0 ? std::min(M, N) : N;
+    int W = 1;
+    for (int w = 2; w <= 8; w *= 2) {
+        const int waves = res * w;
+        if ((128 * w <= E / 8 && waves <= (w == 2 ? 34 : 28)) || (128 * w <= E / 4 && waves <= 8)) W = w;
+    }
+    sh->win = W;
+    sh->wmode = M > 0 ? WIN_TABLE : WIN_PACKED;
+    sh->tbl = std::max(M, 1);
+    sh->stage = 0;
+    sh->stride = layout_stride(1, N);
+    sh->lds = window_lds_bytes(N, M);
+    sh->rpw = 1;
+    sh->block = 64 * W;
+    sh->nblocks = R;
+}
 
 static int launch_shape(int method, int L, int R, LaunchShape *sh) {
     const int N = L * L;
@@ -629,6 +728,7 @@ static int launch_shape(int method, int L, int R, LaunchShape *sh) {
                          "Error: gpu_method %d needs %zu bytes of LDS per workgroup at L=%d (device "
                          "limit %zu); use select_gpu_method",
                          method, sh->lds, L, (size_t)di.lds_block);
+    window_shape(method, L, R, sh);
     return GASP_OK;
 }
 
@@ -676,7 +776,9 @@ static int choose_filter(int method, int L, const LaunchShape &sh, bool mt) {
 struct gasp_engine {
     int L = 0, N = 0, R = 0, method = 0;
     int S = 1, W = 1, stride = 0, rpw = 0, nblocks = 0, block = 0;
-    int tbl = 1;  // sweep_hbm_waves: conflict-table entries
+    int tbl = 1;  // sweep_hbm_waves, sweep_window: table entries
+    int win = 0, wmode = 0;  // sweep_window: waves per replica (0: another kernel) and MODE
+    int layout = 0;  // native layout: 0 bytes, 1 bits, 2 word planes
     size_t lds = 0;
     void *d_lat = nullptr;
     size_t lat_bytes = 0;
@@ -684,7 +786,6 @@ struct gasp_engine {
     float *d_lclus = nullptr;
     int *d_fate = nullptr;
     int *d_counts = nullptr;
-    uint64_t *d_thr = nullptr;
     int8_t *d_spins8 = nullptr;
     int *d_tmp32 = nullptr;
     size_t tmp32_bytes = 0;
@@ -719,12 +820,18 @@ static void engine_free(gasp_engine *e) {
     dfree(e->d_lclus);
     dfree(e->d_fate);
     dfree(e->d_counts);
-    dfree(e->d_thr);
     dfree(e->d_spins8);
     dfree(e->d_tmp32);
     dfree(e->d_draws);
     if (e->stream) (void)hipStreamDestroy(e->stream);
     delete e;
+}
+
+// The engine's sweep kernel at its current shape.
+static SweepFn engine_fn(const gasp_engine *e) {
+    const int rng = e->rng.kind == KIND_MT ? 1 : 0;
+    if (e->win) return window_fn(rng, e->win, e->wmode, is_pow2(e->L), WIN_BITS);
+    return sweep_fn(e->method, rng, e->S, e->W, is_pow2(e->L), e->stage ? e->stage : e->moff);
 }
 
 static int engine_new(int L, int R, int method, gasp_rng_state *d_state, const uint64_t thr[10],
@@ -778,20 +885,23 @@ static int engine_new(int L, int R, int method, gasp_rng_state *d_state, const u
     e->S = sh.S;
     e->W = sh.W;
     e->S0 = e->S;
-    e->adapt = method == 2 && g_tune_slots <= 0;
+    e->win = sh.win;
+    e->wmode = sh.wmode;
+    e->layout = sh.win ? 1 : layout_of(method);
+    e->adapt = method == 2 && g_tune_slots <= 0 && !sh.win;
     e->stride = sh.stride;
     e->ncu = sh.ncu;
     e->lds = sh.lds;
     // the mark plane (if any) lies above the lattice, in the same allocation
-    e->moff = choose_filter(method, L, sh, e->rng.kind == KIND_MT);
+    e->moff = sh.win ? 0 : choose_filter(method, L, sh, e->rng.kind == KIND_MT);
     if (e->moff) e->lds = marks_lds_bytes(e->moff, e->W, e->stride);
     e->tbl = sh.tbl;
     e->stage = sh.stage;
     e->rpw = sh.rpw;
     e->block = sh.block;
     e->nblocks = sh.nblocks;
-    e->lat_bytes = sh.lat_bytes;
-    SweepFn fn = sweep_fn(method, e->rng.kind == KIND_MT ? 1 : 0, e->S, e->W, is_pow2(L), e->stage ? e->stage : e->moff);
+    e->lat_bytes = sh.win ? (size_t)R * sh.stride * 4 : sh.lat_bytes;
+    SweepFn fn = engine_fn(e);
     if (!fn) {
         engine_free(e);
         return set_error(GASP_ERR_ARG, "Error: no kernel for S=%d", e->S);
@@ -811,8 +921,6 @@ static int engine_new(int L, int R, int method, gasp_rng_state *d_state, const u
     ETRY(hipMalloc(&e->d_mag, (size_t)R * sizeof(float)));
     ETRY(hipMalloc(&e->d_fate, (size_t)R * sizeof(int)));
     ETRY(hipMalloc(&e->d_counts, 4 * sizeof(int)));
-    ETRY(hipMalloc(&e->d_thr, 10 * sizeof(uint64_t)));
-    ETRY(hipMemcpyAsync(e->d_thr, e->thr, sizeof e->thr, hipMemcpyHostToDevice, e->stream));
     ETRY(hipMemsetAsync(e->d_fate, 0xff, (size_t)R * sizeof(int), e->stream));  // -1
     ETRY(hipMemsetAsync(e->d_counts, 0, 4 * sizeof(int), e->stream));
     ETRY(hipMemsetAsync(e->d_mag, 0, (size_t)R * sizeof(float), e->stream));
@@ -898,7 +1006,7 @@ static int launch_sweep(gasp_engine *e, uint64_t n_attempts, const uint32_t *dra
     a.n_attempts = n_attempts;
     a.seed = e->rng.seed;
     a.draws = draws;
-    a.thr = e->d_thr;
+    memcpy(a.thr, e->thr, sizeof a.thr);
     a.mag = e->d_mag;
     a.fate = e->d_fate;
     a.counts = e->d_counts;
@@ -907,8 +1015,7 @@ static int launch_sweep(gasp_engine *e, uint64_t n_attempts, const uint32_t *dra
     a.tbl_mask = (unsigned)(e->tbl - 1);
     a.dn_thr = dn;
     a.up_thr = up;
-    SweepFn fn = sweep_fn(e->method, e->rng.kind == KIND_MT ? 1 : 0, e->S, e->W, is_pow2(e->L),
-                          e->stage ? e->stage : e->moff);
+    SweepFn fn = engine_fn(e);
     if (check != CHECK_NONE) {
         hipLaunchKernelGGL(zero_ints, dim3(1), dim3(64), 0, e->stream, e->d_counts, 4);
         HIP_TRY(hipGetLastError());
@@ -975,9 +1082,9 @@ static int engine_set_grids_impl(gasp_engine *e, const int *grids, int on_device
     }
     const int N = e->N, R = e->R, per = R / ninputs;
     const dim3 grid(1024), blk(256);
-    if (layout_of(e->method) == 2) {
+    if (e->layout == 2) {
         hipLaunchKernelGGL(pack_multispin, grid, blk, 0, e->stream, src, (unsigned *)e->d_lat, R, N, e->stride, per);
-    } else if (e->method == 1) {
+    } else if (e->layout == 1) {
         hipLaunchKernelGGL(pack_bits, grid, blk, 0, e->stream, src, (unsigned *)e->d_lat, R, N, e->stride, per);
     } else {
         hipLaunchKernelGGL(pack_hbm, grid, blk, 0, e->stream, src, (unsigned char *)e->d_lat, R, N, e->stride, per);
@@ -990,10 +1097,10 @@ template <typename T>
 static int engine_unpack(gasp_engine *e, T *dst) {
     const int N = e->N, R = e->R;
     const dim3 grid(1024), blk(256);
-    if (layout_of(e->method) == 2) {
+    if (e->layout == 2) {
         hipLaunchKernelGGL(unpack_multispin<T>, grid, blk, 0, e->stream, (const unsigned *)e->d_lat, dst, R, N,
                            e->stride);
-    } else if (e->method == 1) {
+    } else if (e->layout == 1) {
         hipLaunchKernelGGL(unpack_bits<T>, grid, blk, 0, e->stream, (const unsigned *)e->d_lat, dst, R, N, e->stride);
     } else {
         hipLaunchKernelGGL(unpack_hbm<T>, grid, blk, 0, e->stream, (const unsigned char *)e->d_lat, dst, R, N,
@@ -1185,7 +1292,7 @@ extern "C" int gasp_engine_get_gridstates(gasp_engine *e, uint8_t *host_out) {
     uint8_t *d = nullptr;
     hipError_t he = hipMalloc(&d, nbytes);
     if (he == hipSuccess) {
-        hipLaunchKernelGGL(pack_gridstates, dim3(2048), dim3(256), 0, e->stream, (const void *)e->d_lat, layout_of(e->method),
+        hipLaunchKernelGGL(pack_gridstates, dim3(2048), dim3(256), 0, e->stream, (const void *)e->d_lat, e->layout,
                            e->stride, e->R, e->N, d, nbytes);
         he = hipGetLastError();
     }
@@ -1214,7 +1321,7 @@ extern "C" int gasp_engine_gather_grids(gasp_engine *e, const int *replicas, int
     if (he == hipSuccess) he = hipMalloc(&d_out, bytes);
     if (he == hipSuccess) he = hipMemcpyAsync(d_idx, replicas, (size_t)n * sizeof(int), hipMemcpyHostToDevice, e->stream);
     if (he == hipSuccess) {
-        hipLaunchKernelGGL(gather_spins8, dim3(1024), dim3(256), 0, e->stream, (const void *)e->d_lat, layout_of(e->method),
+        hipLaunchKernelGGL(gather_spins8, dim3(1024), dim3(256), 0, e->stream, (const void *)e->d_lat, e->layout,
                            e->stride, d_idx, n, e->N, d_out);
         he = hipGetLastError();
     }
@@ -1312,7 +1419,7 @@ extern "C" int gasp_engine_get_conflict_filter(gasp_engine *e, int *filter) {
 
 extern "C" int gasp_engine_get_lattice_staging(gasp_engine *e, int *staging) {
     if (!e || !staging) return set_error(GASP_ERR_ARG, "gasp_engine_get_lattice_staging: NULL argument");
-    *staging = e->stage + 1;
+    *staging = e->win && e->method == 0 ? 3 : e->stage + 1;  // sweep_window: spins in LDS, one bit each
     return GASP_OK;
 }
 
@@ -1328,22 +1435,8 @@ extern "C" int gasp_engine_get_lattice_staging(gasp_engine *e, int *staging) {
 // magnetisation when the caller passes none (256: R floats) and the native
 // lattice.
 
-// Stores the thresholds and clears the counters (a kernel rather than a host
-// copy or a memset, so that the sequence can be captured and replayed).
-struct Thresholds10 {
-    uint64_t v[10];
-};
-__global__ void set_thresholds(Thresholds10 t, uint64_t *thr, int *counts) {
-    const int i = threadIdx.x;
-    if (i < 10) thr[i] = t.v[i];
-    if (i < 4) counts[i] = 0;
-}
-
 static size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 
-static size_t grids_ws_lattice_offset(int R, bool own_mag) {
-    return own_mag ? align256(256 + (size_t)R * sizeof(float)) : 256;
-}
 
 static int grids_check_args(int L, int R, int method, gasp_rng_state *d_state, const int *d_grids, int nsweeps) {
     if (L < 2 || L > 8192) return set_error(GASP_ERR_ARG, "Error: L must lie in [2, 8192]");
@@ -1355,34 +1448,32 @@ static int grids_check_args(int L, int R, int method, gasp_rng_state *d_state, c
     return GASP_OK;
 }
 
-// The workspace must hold grids_ws_lattice_offset(R, !d_mag) + sh.lat_bytes.
+// The workspace holds the magnetisation when the caller passes none, then
+// (at the next multiple of 256 bytes) the native lattice unless the kernel
+// works on the caller's grids.
 static int sweep_grids_run(int L, int R, int method, gasp_rng_state *d_state, double beta, double h, int *d_grids,
                            int nsweeps, float *d_mag, hipStream_t st, const LaunchShape &sh, unsigned char *ws) {
     const int N = L * L;
+    SweepArgs a{};
     float pf[20];
-    Thresholds10 t;
     table_f32(beta, h, pf);
-    thr_from_table_f(pf, t.v);
-    uint64_t *d_thr = (uint64_t *)ws;
-    int *d_counts = (int *)(ws + 128);
-    float *mag = d_mag ? d_mag : (float *)(ws + 256);
-    void *lat = ws + grids_ws_lattice_offset(R, !d_mag);
-    hipLaunchKernelGGL(set_thresholds, dim3(1), dim3(64), 0, st, t, d_thr, d_counts);
-    HIP_TRY(hipGetLastError());
+    thr_from_table_f(pf, a.thr);
+    float *mag = d_mag ? d_mag : (float *)ws;
+    void *lat = sh.win ? (void *)d_grids : ws + (d_mag ? 0 : align256((size_t)R * sizeof(float)));
     const dim3 grid(1024), blk(256);
-    const int lay = layout_of(method);
+    const int lay = sh.win ? -1 : layout_of(method);  // sweep_window works on the caller's grids
     if (lay == 2)
         hipLaunchKernelGGL(pack_multispin, grid, blk, 0, st, d_grids, (unsigned *)lat, R, N, sh.stride, 1);
     else if (lay == 1)
         hipLaunchKernelGGL(pack_bits, grid, blk, 0, st, d_grids, (unsigned *)lat, R, N, sh.stride, 1);
-    else
+    else if (lay == 0)
         hipLaunchKernelGGL(pack_hbm, grid, blk, 0, st, d_grids, (unsigned char *)lat, R, N, sh.stride, 1);
     HIP_TRY(hipGetLastError());
-    SweepFn fn = sweep_fn(method, 0, sh.S, sh.W, is_pow2(L), sh.stage);
+    SweepFn fn = sh.win ? window_fn(0, sh.win, sh.wmode, is_pow2(L), WIN_INT32)
+                        : sweep_fn(method, 0, sh.S, sh.W, is_pow2(L), sh.stage);
     if (!fn) return set_error(GASP_ERR_ARG, "Error: no kernel for S=%d", sh.S);
     if (sh.lds > 65536)
         HIP_TRY(hipFuncSetAttribute((const void *)fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)sh.lds));
-    SweepArgs a{};
     a.lattice = lat;
     a.L = L;
     a.N = N;
@@ -1391,9 +1482,7 @@ static int sweep_grids_run(int L, int R, int method, gasp_rng_state *d_state, do
     a.rpw = sh.rpw;
     a.stride = sh.stride;
     a.rng_dev = (const RngHeader *)d_state;
-    a.thr = d_thr;
     a.mag = mag;
-    a.counts = d_counts;
     a.check = CHECK_NONE;
     a.tbl_mask = (unsigned)(sh.tbl - 1);
     // launches of at most 2^30 attempts per replica (32-bit launch-local
@@ -1414,7 +1503,7 @@ static int sweep_grids_run(int L, int R, int method, gasp_rng_state *d_state, do
         hipLaunchKernelGGL(unpack_multispin<int>, grid, blk, 0, st, (const unsigned *)lat, d_grids, R, N, sh.stride);
     else if (lay == 1)
         hipLaunchKernelGGL(unpack_bits<int>, grid, blk, 0, st, (const unsigned *)lat, d_grids, R, N, sh.stride);
-    else
+    else if (lay == 0)
         hipLaunchKernelGGL(unpack_hbm<int>, grid, blk, 0, st, (const unsigned char *)lat, d_grids, R, N, sh.stride);
     HIP_TRY(hipGetLastError());
     return GASP_OK;
@@ -1428,14 +1517,15 @@ extern "C" int gasp_sweep_grids(int L, int ngrids, int gpu_method, gasp_rng_stat
     LaunchShape sh;
     if ((rc = launch_shape(gpu_method, L, ngrids, &sh))) return rc;
     hipStream_t st = (hipStream_t)stream;
-    const size_t bytes = grids_ws_lattice_offset(ngrids, !d_mag) + sh.lat_bytes;
+    // sweep_window works on the caller's grids: no native lattice
+    const size_t bytes = (d_mag ? 0 : align256((size_t)ngrids * sizeof(float))) + (sh.win ? 0 : sh.lat_bytes);
     unsigned char *ws = nullptr;
-    hipError_t he = hipMallocAsync((void **)&ws, bytes, st);
+    hipError_t he = bytes ? hipMallocAsync((void **)&ws, bytes, st) : hipSuccess;
     if (he != hipSuccess)
         return set_error(he == hipErrorOutOfMemory ? GASP_ERR_NOMEM : GASP_ERR_HIP, "GPUassert: %s %s %d",
                          hipGetErrorString(he), __FILE__, __LINE__);
     rc = sweep_grids_run(L, ngrids, gpu_method, d_state, beta, h, d_ising_grids, nsweeps, d_mag, st, sh, ws);
-    he = hipFreeAsync(ws, st);
+    he = ws ? hipFreeAsync(ws, st) : hipSuccess;
     if (!rc && he != hipSuccess)
         rc = set_error(GASP_ERR_HIP, "GPUassert: %s %s %d", hipGetErrorString(he), __FILE__, __LINE__);
     return rc;
@@ -1478,7 +1568,8 @@ extern "C" int gasp_sweep_grids_noalloc(int L, int ngrids, int gpu_method, gasp_
     if (rc) return rc;
     LaunchShape sh;
     if ((rc = launch_shape(gpu_method, L, ngrids, &sh))) return rc;
-    const size_t bytes = grids_ws_lattice_offset(ngrids, !d_mag) + sh.lat_bytes;
+    // the refusal counts the method's native lattice whichever kernel runs
+    const size_t bytes = (d_mag ? 256 : align256(256 + (size_t)ngrids * sizeof(float))) + sh.lat_bytes;
     if (bytes > kSweepScratchBytes)
         return set_error(GASP_ERR_ARG,
                          "gasp_sweep_grids_noalloc: gpu_method %d with L=%d, ngrids=%d needs %zu bytes of "
@@ -1823,10 +1914,29 @@ extern "C" int gasp_autotune(int method, int L, int ngrids, double beta, double 
             bw = W;
         }
     }
+    // sweep_window, which no (S, W) names, where the automatic choice takes it
+    bool window = false;
+    g_tuned.erase(std::make_tuple(method, L, ngrids));
+    g_tune_slots = g_tune_waves = 0;
+    {
+        gasp_engine *e = nullptr;
+        if (!engine_new(L, ngrids, method, rng, thr, 0, beta, h, &e)) {
+            if (e->win) {
+                const double rate = probe_rate(e, grids, ngrids, probe_sweeps, probe_sweeps);
+                window = rate > best;
+                best = std::max(rate, best);
+            }
+            engine_free(e);
+        } else {
+            clear_error();
+        }
+    }
     int blaunch = check_sweeps;
     if (best > 0 && check_sweeps > 1) {
-        g_tune_slots = bs;
-        g_tune_waves = bw;
+        if (!window) {
+            g_tune_slots = bs;
+            g_tune_waves = bw;
+        }
         gasp_engine *e = nullptr;
         if (!engine_new(L, ngrids, method, rng, thr, 0, beta, h, &e)) {
             double best_l = -1.0;
@@ -1847,7 +1957,7 @@ extern "C" int gasp_autotune(int method, int L, int ngrids, double beta, double 
     g_tune_waves = save_w;
     (void)hipFree(rng);
     if (best < 0) return set_error(GASP_ERR_ARG, "gasp_autotune: no candidate ran");
-    g_tuned[std::make_tuple(method, L, ngrids)] = {bs, bw};
+    g_tuned[std::make_tuple(method, L, ngrids)] = {bs, bw, window};
     if (best_slots) *best_slots = bs;
     if (best_waves) *best_waves = bw;
     if (best_launch_sweeps) *best_launch_sweeps = blaunch;
@@ -2037,7 +2147,7 @@ extern "C" void mc_driver_gpu(mc_gpu_grids_t grids, double beta, double h, int *
             if ((rc = engine_check_cv(e, e->d_lclus, check_mode, dn, up))) break;
         }
         if (do_grid && packed_out) {
-            hipLaunchKernelGGL(pack_gridstates, dim3(2048), dim3(256), 0, e->stream, (const void *)e->d_lat, layout_of(e->method),
+            hipLaunchKernelGGL(pack_gridstates, dim3(2048), dim3(256), 0, e->stream, (const void *)e->d_lat, e->layout,
                                e->stride, R, e->N, d_bits, pbytes);
             if (hipGetLastError() != hipSuccess ||
                 hipMemcpyAsync(h_bits, d_bits, pbytes, hipMemcpyDeviceToHost, e->stream) != hipSuccess) {

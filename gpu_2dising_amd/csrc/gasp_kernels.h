@@ -104,7 +104,7 @@ struct SweepArgs {
     uint64_t n_attempts;     // attempts per replica in this launch (< 2^31)
     uint64_t seed;           // Philox key
     const uint32_t *draws;   // RNG_DRAWS: [R][3*n_attempts], draw stream from a_begin
-    const uint64_t *thr;     // 10 thresholds, j = 5*s01 + (number of up neighbours)
+    uint64_t thr[10];        // thresholds, j = 5*s01 + (number of up neighbours)
     float *mag;              // out: magnetisation per replica
     int *fate;               // CHECK_FATES: fates per replica
     int *counts;             // out: [0] #(m>up), [1] #fate 0, [2] #fate 1

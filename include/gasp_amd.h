@@ -221,6 +221,13 @@ void gasp_free(void *d_ptr);
  * 1 and 2: up to 64.  Method 3 (bit-sliced, below): the first value is the number of
  * waves per workgroup (1, 2, 4 or 8) that evaluate one word group's attempts
  * together, the second the word split (1: 64 replicas per word, 2: 32).
+ * With both 0, methods 0 to 2 with few replicas (up to 64 per CU at small L, 40
+ * at large L; method 0 from L = 32 on always) run one replica per workgroup on
+ * a kernel of its own that no (slots, waves) names; gasp_get_tuning and
+ * gasp_engine_get_shape then report what the method's other kernels would
+ * take.  Any explicit value here, and gasp_set_conflict_filter,
+ * gasp_set_lattice_staging and gasp_set_dependence_tables, keep the kernels
+ * that they describe.  Trajectories do not depend on the choice.
  * Applies to subsequent runs. */
 void gasp_set_tuning(int slots_per_replica, int waves_per_group);
 void gasp_get_tuning(int method, int L, int ngrids, int *slots_per_replica,
@@ -338,8 +345,9 @@ int gasp_engine_largest_cluster(gasp_engine *e, int spin, float *host_out);
  * successive calls continue each replica's chain and nothing is read back to
  * the host (a state of the wrong kind leaves the grids alone and writes NaN
  * magnetisations).  The work is queued on `stream` (a hipStream_t; NULL: the
- * null stream) and not waited for.  Allocates (stream-ordered) a workspace
- * of about the method's native lattice for each call. */
+ * null stream) and not waited for.  With few replicas (see gasp_set_tuning)
+ * the sweep kernel reads and writes d_ising_grids itself; else the call
+ * allocates (stream-ordered) a workspace of about the method's native lattice. */
 int gasp_sweep_grids(int L, int ngrids, int gpu_method, gasp_rng_state *d_state, double beta, double h,
                      int *d_ising_grids, int nsweeps, float *d_mag, void *stream);
 /* No counterpart in the reference: for callers that cannot allocate device
@@ -374,7 +382,8 @@ int gasp_engine_set_attempt(gasp_engine *e, unsigned long long attempt);
  * engines without the choice). */
 int gasp_engine_get_conflict_filter(gasp_engine *e, int *filter);
 /* The engine's lattice staging, as gasp_set_lattice_staging takes it (1 for
- * engines without the choice). */
+ * engines without the choice; 3 for a method-0 engine on the kernel of one
+ * replica per workgroup, which keeps the spins in LDS). */
 int gasp_engine_get_lattice_staging(gasp_engine *e, int *staging);
 
 /* ------------------------------------------------ batched graph, autotuner */
