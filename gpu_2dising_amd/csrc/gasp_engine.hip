@@ -1053,7 +1053,7 @@ static int engine_advance(gasp_engine *e, uint64_t n, int check, double dn, doub
         const uint64_t nb = std::min(left, cap);
         if (e->rng.kind == KIND_MT) {
             uint32_t *st = (uint32_t *)((char *)e->d_rng + kRngMtOffset);
-            hipLaunchKernelGGL(mt_draws_kernel, dim3(e->R), dim3(64), 0, e->stream, st, e->R,
+            hipLaunchKernelGGL(mt_draws_kernel, dim3(e->R), dim3(256), 0, e->stream, st, e->R,
                                3ull * e->rng.attempts, 3ull * nb, e->d_draws);
             HIP_TRY(hipGetLastError());
         }
