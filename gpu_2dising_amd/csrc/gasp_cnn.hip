@@ -631,6 +631,8 @@ __global__ void gather_batch(const int8_t *__restrict__ data, const float *__res
 
 }  // namespace cnn
 
+#include "gasp_cnn_stream.h"
+
 using namespace cnn;
 
 // =================================================================== host side
@@ -645,6 +647,13 @@ struct gasp_cnn {
     uint16_t *dz0 = nullptr, *dz1 = nullptr;
     float *part = nullptr, *part1 = nullptr, *part_head = nullptr;
     float *red = nullptr;  // chunk sums of the two-level reductions
+    bool stream = false;   // L <= 64: whole images through a workgroup (gasp_cnn_stream.h)
+    int ncu = 256;
+    uint16_t *tab = nullptr;            // conv1's table
+    uint32_t *m4 = nullptr;             // a4 > 0, a bit per channel
+    uint16_t *code = nullptr;           // every position's row of conv1's table
+    float *pool = nullptr;              // net_fwd's sums of a4
+    float *parts[5] = {nullptr, nullptr, nullptr, nullptr, nullptr};  // parts[2..4]: weight-gradient partials
     int8_t *data = nullptr;
     float *data_y = nullptr;
     int *order = nullptr;
@@ -673,11 +682,29 @@ extern "C" int gasp_cnn_destroy(gasp_cnn *c) {
                     (void *)c->wb, (void *)c->s, (void *)c->y, (void *)c->pb, (void *)c->loss, (void *)c->dg,
                     (void *)c->a[1], (void *)c->a[2], (void *)c->a[3], (void *)c->a[4], (void *)c->dz0,
                     (void *)c->dz1, (void *)c->part, (void *)c->part1, (void *)c->part_head,
-                    (void *)c->red, (void *)c->data, (void *)c->data_y, (void *)c->order})
+                    (void *)c->red, (void *)c->data, (void *)c->data_y, (void *)c->order, (void *)c->tab, (void *)c->m4, (void *)c->code,
+                    (void *)c->pool, (void *)c->parts[2], (void *)c->parts[3], (void *)c->parts[4]})
         cfree(q);
     if (c->st) (void)hipStreamDestroy(c->st);
     delete c;
     return GASP_OK;
+}
+
+// The streamed kernels take more than 64 KB of LDS.
+template <int LG>
+static hipError_t net_attributes() {
+    constexpr int L = 1 << LG;
+    const struct {
+        const void *f;
+        int lds;
+    } fns[] = {{(const void *)net_fwd<false, LG>, kFwdLds}, {(const void *)net_fwd<true, LG>, kFwdLds},
+               {(const void *)net_back<4, LG>, back_lds(L)}, {(const void *)net_back<3, LG>, back_lds(L)},
+               {(const void *)net_back<2, LG>, back_lds(L)}};
+    for (const auto &f : fns) {
+        const hipError_t e = hipFuncSetAttribute(f.f, hipFuncAttributeMaxDynamicSharedMemorySize, f.lds);
+        if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
 }
 
 extern "C" int gasp_cnn_create(int L, int max_batch, gasp_cnn **out) {
@@ -708,13 +735,28 @@ extern "C" int gasp_cnn_create(int L, int max_batch, gasp_cnn **out) {
     A((void **)&c->pb, n * 4);
     A((void **)&c->loss, n * 4);
     A((void **)&c->dg, n * C * 4);
-    for (int k = 1; k <= 4; ++k) A((void **)&c->a[k], n * N * C * 2);
+    A((void **)&c->a[2], n * N * C * 2);
+    A((void **)&c->a[3], n * N * C * 2);
     A((void **)&c->dz0, n * N * C * 2);
     A((void **)&c->dz1, n * N * C * 2);
-    A((void **)&c->part, n * 4 * kWgRow * 4);
-    A((void **)&c->part1, n * (size_t)L * 320 * 4);
     A((void **)&c->part_head, n * HEAD_N * 4);
-    {
+    c->stream = L <= 64;
+    int dev = 0;
+    if (e == hipSuccess) e = hipGetDevice(&dev);
+    if (e == hipSuccess) e = hipDeviceGetAttribute(&c->ncu, hipDeviceAttributeMultiprocessorCount, dev);
+    if (c->stream) {
+        A((void **)&c->tab, 512 * C * 2);
+        A((void **)&c->m4, n * N * 4);
+        A((void **)&c->code, n * N * 2);
+        A((void **)&c->pool, ((n * L + 63) / 64) * (size_t)std::max(1, L / 8) * 4 * (64 / L) * C * 4);
+        for (int k = 2; k <= 4; ++k) A((void **)&c->parts[k], std::min<size_t>(kWgBlocks, n * 4) * kWgRow * 4);
+        A((void **)&c->part1, std::min<size_t>(kW1Blocks, n * L) * 320 * 4);
+        if (e == hipSuccess) e = L == 64 ? net_attributes<6>() : L == 32 ? net_attributes<5>() : net_attributes<4>();
+    } else {
+        A((void **)&c->a[1], n * N * C * 2);
+        A((void **)&c->a[4], n * N * C * 2);
+        A((void **)&c->part, n * 4 * kWgRow * 4);
+        A((void **)&c->part1, n * (size_t)L * 320 * 4);
         const size_t q = (size_t)kRedChunk;
         const size_t r = std::max({(n * 4 + q - 1) / q * kWgRow, (n * L + q - 1) / q * 320, (n + q - 1) / q * HEAD_N});
         A((void **)&c->red, r * 4);
@@ -774,8 +816,97 @@ extern "C" int gasp_cnn_get_params(gasp_cnn *c, float *host_params) {
     return GASP_OK;
 }
 
+// net_fwd's units for n images: the fewest steps (blocks of the busiest
+// workgroup and the pipeline's four) over bands of 8 rows or more.
+static NetShape net_shape(const gasp_cnn *c, int n) {
+    NetShape g{};
+    g.n = n;
+    const int groups = (n * c->L + 63) / 64;
+    long long best = 0;
+    for (int nb = 1; nb == 1 || c->L / nb >= 8; nb *= 2) {
+        const long long units = (long long)groups * nb;
+        const long long steps = ((units + c->ncu - 1) / c->ncu) * (c->L / nb / 4 + 1) + 4;
+        if (nb == 1 || steps < best) {
+            best = steps;
+            g.nb = nb;
+        }
+    }
+    g.Rb = c->L / g.nb;
+    g.units = groups * g.nb;
+    return g;
+}
+
+// pb[0 .. n) from s[0 .. n)
+template <int LG>
+static int infer_stream(gasp_cnn *c, const int8_t *s, int n, float *pb) {
+    const NetShape g = net_shape(c, n);
+    hipLaunchKernelGGL((net_fwd<false, LG>), dim3(std::min(g.units, c->ncu)), dim3(kFwdThreads), kFwdLds, c->st, s, c->wf, c->p,
+                       c->w1r, (uint16_t *)nullptr, (uint16_t *)nullptr, (uint16_t *)nullptr, (uint32_t *)nullptr, c->pool,
+                       (uint16_t *)nullptr, (uint16_t *)nullptr, g);
+    hipLaunchKernelGGL((net_head<false, LG>), dim3(n), dim3(64), 0, c->st, c->pool, c->p, (const float *)nullptr, pb, c->loss,
+                       c->part_head, c->dg, g, 0.0f);
+    CTRY(hipGetLastError());
+    return GASP_OK;
+}
+template <int LG>
+static int forward_stream(gasp_cnn *c, int n, const float *d_labels) {
+    if (!d_labels) return infer_stream<LG>(c, c->s, n, c->pb);
+    const NetShape g = net_shape(c, n);
+    const dim3 grid(std::min(g.units, c->ncu));
+    // Training adds the pooled features up row after row as `head` does.  Where
+    // few images make bands worth it (37 of L = 32: 30 us against 38), the
+    // bands' sums would be added in another order: a4 goes to memory instead (in
+    // dz1, free until net_back<3>) and `head` pools it.
+    uint16_t *a4 = g.nb > 1 ? c->dz1 : nullptr;
+    hipLaunchKernelGGL((net_fwd<true, LG>), grid, dim3(kFwdThreads), kFwdLds, c->st, c->s, c->wf, c->p, c->w1r, c->a[2],
+                       c->a[3], a4, c->m4, c->pool, c->tab, c->code, g);
+    if (a4)
+        hipLaunchKernelGGL(head, dim3(n), dim3(256), 0, c->st, a4, c->p, d_labels, c->pb, c->loss, c->part_head, c->dg, n,
+                           c->L, 1.0f / (float)n);
+    else
+        hipLaunchKernelGGL((net_head<true, LG>), dim3(n), dim3(64), 0, c->st, c->pool, c->p, d_labels, c->pb, c->loss,
+                           c->part_head, c->dg, g, 1.0f / (float)n);
+    CTRY(hipGetLastError());
+    return GASP_OK;
+}
+
+// backward after forward_stream(c, n, labels): fills c->g, and with `ad` takes the
+// Adam step
+template <int LG>
+static int backward_stream(gasp_cnn *c, int n, const AdamArgs *ad) {
+    constexpr int L = 1 << LG;
+    const int bands = n * (L / 4);
+    const int chains = std::min({bands, kWgBlocks, 4 * c->nmax});  // partial rows (see backward)
+    const dim3 grid(std::min(chains, c->ncu)), blk(kBackThreads);
+    constexpr size_t W = 9 * 2 * 64 * 8;
+    hipLaunchKernelGGL((net_back<4, LG>), grid, blk, back_lds(L), c->st, (const uint16_t *)nullptr, c->m4, c->dg, c->a[3],
+                       (const uint16_t *)nullptr, c->wb + 2 * W, c->dz0, c->parts[4], bands, chains);
+    hipLaunchKernelGGL((net_back<3, LG>), grid, blk, back_lds(L), c->st, c->dz0, (const uint32_t *)nullptr,
+                       (const float *)nullptr, c->a[2], (const uint16_t *)nullptr, c->wb + W, c->dz1, c->parts[3], bands, chains);
+    hipLaunchKernelGGL((net_back<2, LG>), grid, blk, back_lds(L), c->st, c->dz1, (const uint32_t *)nullptr,
+                       (const float *)nullptr, c->tab, c->code, c->wb, c->dz0, c->parts[2], bands, chains);
+    const int n1 = std::min({bands, kW1Blocks, n * L});
+    hipLaunchKernelGGL(conv1_wgrad, dim3(n1), dim3(256), 0, c->st, c->s, c->dz0, c->part1, n, L);
+    const NetParts q = {{c->part1, c->parts[2], c->parts[3], c->parts[4], c->part_head}, {n1, chains, chains, chains, n}};
+    if (ad)
+        hipLaunchKernelGGL(net_reduce<true>, dim3(kRedBlocks), dim3(kRedThreads), 0, c->st, q, c->g, c->p, c->m, c->v, c->wf,
+                           c->wb, c->w1r, *ad);
+    else
+        hipLaunchKernelGGL(net_reduce<false>, dim3(kRedBlocks), dim3(kRedThreads), 0, c->st, q, c->g, c->p, c->m, c->v, c->wf,
+                           c->wb, c->w1r, AdamArgs{});
+    CTRY(hipGetLastError());
+    return GASP_OK;
+}
+static int backward_stream(gasp_cnn *c, int n, const AdamArgs *ad) {
+    return c->L == 64 ? backward_stream<6>(c, n, ad) : c->L == 32 ? backward_stream<5>(c, n, ad) : backward_stream<4>(c, n, ad);
+}
+
 // forward of n <= nmax grids already in c->s
 static int forward(gasp_cnn *c, int n, const float *d_labels) {
+    if (c->stream)
+        return c->L == 64   ? forward_stream<6>(c, n, d_labels)
+               : c->L == 32 ? forward_stream<5>(c, n, d_labels)
+                            : forward_stream<4>(c, n, d_labels);
     const int L = c->L, N = c->N;
     const size_t tot = (size_t)n * N;
     hipLaunchKernelGGL(conv1_fwd, dim3((unsigned)((tot + 255) / 256)), dim3(256), 0, c->st, c->s, c->w1r, c->p,
@@ -793,6 +924,7 @@ static int forward(gasp_cnn *c, int n, const float *d_labels) {
 
 // backward after forward(c, n, labels): fills c->g
 static int backward(gasp_cnn *c, int n) {
+    if (c->stream) return backward_stream(c, n, nullptr);
     const int L = c->L, N = c->N;
     const size_t tot = (size_t)n * N;
     const int rows = n * L;
@@ -866,10 +998,17 @@ extern "C" int gasp_cnn_gradient(gasp_cnn *c, const int8_t *spins, const float *
     return GASP_OK;
 }
 
-static int adam_step(gasp_cnn *c, float lr) {
+// backward and the Adam step
+static int backward_adam(gasp_cnn *c, int n, float lr) {
     c->step++;
     const float b1 = 0.9f, b2 = 0.999f;
     const float c1 = 1.0f - powf(b1, (float)c->step), c2 = 1.0f - powf(b2, (float)c->step);
+    if (c->stream) {
+        const AdamArgs ad = {lr, b1, b2, 1e-8f, c1, c2};
+        return backward_stream(c, n, &ad);
+    }
+    const int rc = backward(c, n);
+    if (rc) return rc;
     hipLaunchKernelGGL(adam, dim3((NPARAM + 255) / 256), dim3(256), 0, c->st, c->p, c->g, c->m, c->v, NPARAM, lr, b1,
                        b2, 1e-8f, c1, c2);
     CTRY(hipGetLastError());
@@ -884,8 +1023,7 @@ extern "C" int gasp_cnn_train_step(gasp_cnn *c, const int8_t *spins, const float
     if (!c->weights_ready) return set_error(GASP_ERR_ARG, "gasp_cnn_train_step: parameters not set");
     int rc = load_batch(c, spins, labels, n);
     if (!rc) rc = forward(c, n, c->y);
-    if (!rc) rc = backward(c, n);
-    if (!rc) rc = adam_step(c, lr);
+    if (!rc) rc = backward_adam(c, n, lr);
     if (rc) return rc;
     std::vector<float> l(n);
     CTRY(hipMemcpyAsync(l.data(), c->loss, (size_t)n * 4, hipMemcpyDeviceToHost, c->st));
@@ -934,8 +1072,7 @@ extern "C" int gasp_cnn_train_epoch(gasp_cnn *c, const int *order, int count, in
         hipLaunchKernelGGL(gather_batch, dim3((unsigned)((words + 255) / 256)), dim3(256), 0, c->st, c->data,
                            c->data_y, c->order + i0, nb, c->N, c->s, c->y);
         int rc = forward(c, nb, c->y);
-        if (!rc) rc = backward(c, nb);
-        if (!rc) rc = adam_step(c, lr);
+        if (!rc) rc = backward_adam(c, nb, lr);
         if (rc) return rc;
         CTRY(hipMemcpyAsync(l.data(), c->loss, (size_t)nb * 4, hipMemcpyDeviceToHost, c->st));
         CTRY(hipStreamSynchronize(c->st));
