@@ -193,6 +193,7 @@ __global__ void __launch_bounds__(64 * W) sweep_window(SweepArgs a) {
     uint32_t uaA = 0u, uaB = 0u;
     uint32_t nxt = min(S, NP), ndef = 0u, left = kRounds;
     bool hold = false;
+    uint32_t ahead = 0u;
     for (;;) {
         if (__builtin_amdgcn_inverse_ballot_w64(fresh)) {
             if constexpr (RNG == RNG_PHILOX) {
@@ -216,6 +217,15 @@ __global__ void __launch_bounds__(64 * W) sweep_window(SweepArgs a) {
                 sA = geo.mt(u0, u1);
                 sB = geo.mt(v0, v1);
             }
+        }
+        if constexpr (RNG == RNG_DRAWS) {
+            // The draws of a pair are 24 bytes that no earlier round has loaded:
+            // touch those of the pairs after next round's (a load every 64
+            // bytes), so that a round finds its own in the cache.  100 sweeps of
+            // 256 replicas at L = 32: 0.97 -> 0.70 ms.
+            asm volatile("" ::"v"(ahead));
+            const uint64_t at = 6ull * (nxt + S) + 16ull * (uint32_t)tid;
+            if (at < 6ull * (nxt + 2u * S) && at < 3ull * a.n_attempts) ahead = drw[at];
         }
         // the pair's keys (B's is one more); MODE 0 keeps the spin below them
         const uint32_t base = (left << kWinIdxBits) - 2u * (nxt - kWinSpan);
