@@ -786,7 +786,6 @@ struct gasp_engine {
     float *d_lclus = nullptr;
     int *d_fate = nullptr;
     int *d_counts = nullptr;
-    int8_t *d_spins8 = nullptr;
     int *d_tmp32 = nullptr;
     size_t tmp32_bytes = 0;
     int freeze = 0;          // skip replicas whose fate is decided
@@ -820,7 +819,6 @@ static void engine_free(gasp_engine *e) {
     dfree(e->d_lclus);
     dfree(e->d_fate);
     dfree(e->d_counts);
-    dfree(e->d_spins8);
     dfree(e->d_tmp32);
     dfree(e->d_draws);
     if (e->stream) (void)hipStreamDestroy(e->stream);
@@ -1067,25 +1065,37 @@ static int engine_advance(gasp_engine *e, uint64_t n, int check, double dn, doub
 
 // Packs int32 grids into the native layout.  `ninputs` grids are given;
 // replica r takes grid r / (R / ninputs) (ninputs == R: one grid per replica).
+static size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
+
+// The engine's scratch memory, at least `bytes`: staging of grids, packed records
+// and gathered replicas between the native layout and the host (kept until the
+// engine is destroyed; work on it is ordered by the engine's stream).
+static hipError_t engine_scratch(gasp_engine *e, size_t bytes) {
+    if (e->d_tmp32 && e->tmp32_bytes >= bytes) return hipSuccess;
+    dfree(e->d_tmp32);
+    e->d_tmp32 = nullptr;
+    e->tmp32_bytes = bytes;
+    return hipMalloc(&e->d_tmp32, bytes);
+}
+static int scratch_error(hipError_t he) {
+    return set_error(he == hipErrorOutOfMemory ? GASP_ERR_NOMEM : GASP_ERR_HIP, "GPUassert: %s %s %d",
+                     hipGetErrorString(he), __FILE__, __LINE__);
+}
+
 static int engine_set_grids_impl(gasp_engine *e, const int *grids, int on_device, int ninputs) {
     const size_t bytes = (size_t)ninputs * e->N * sizeof(int);
     const int *src = grids;
     if (!on_device) {
-        if (!e->d_tmp32 || e->tmp32_bytes < bytes) {
-            dfree(e->d_tmp32);
-            e->d_tmp32 = nullptr;
-            HIP_TRY(hipMalloc(&e->d_tmp32, bytes));
-            e->tmp32_bytes = bytes;
-        }
+        HIP_TRY(engine_scratch(e, bytes));
         HIP_TRY(hipMemcpyAsync(e->d_tmp32, grids, bytes, hipMemcpyHostToDevice, e->stream));
         src = e->d_tmp32;
     }
     const int N = e->N, R = e->R, per = R / ninputs;
     const dim3 grid(1024), blk(256);
     if (e->layout == 2) {
-        hipLaunchKernelGGL(pack_multispin, grid, blk, 0, e->stream, src, (unsigned *)e->d_lat, R, N, e->stride, per);
+        hipLaunchKernelGGL(pack_multispin, dim3(4096), blk, 0, e->stream, src, (unsigned *)e->d_lat, R, N, e->stride, per);
     } else if (e->layout == 1) {
-        hipLaunchKernelGGL(pack_bits, grid, blk, 0, e->stream, src, (unsigned *)e->d_lat, R, N, e->stride, per);
+        hipLaunchKernelGGL(pack_bits, bits_grid(R, 32 * e->stride), blk, 0, e->stream, src, (unsigned *)e->d_lat, R, N, e->stride, per);
     } else {
         hipLaunchKernelGGL(pack_hbm, grid, blk, 0, e->stream, src, (unsigned char *)e->d_lat, R, N, e->stride, per);
     }
@@ -1098,10 +1108,10 @@ static int engine_unpack(gasp_engine *e, T *dst) {
     const int N = e->N, R = e->R;
     const dim3 grid(1024), blk(256);
     if (e->layout == 2) {
-        hipLaunchKernelGGL(unpack_multispin<T>, grid, blk, 0, e->stream, (const unsigned *)e->d_lat, dst, R, N,
+        hipLaunchKernelGGL(unpack_multispin<T>, dim3(4096), blk, 0, e->stream, (const unsigned *)e->d_lat, dst, R, N,
                            e->stride);
     } else if (e->layout == 1) {
-        hipLaunchKernelGGL(unpack_bits<T>, grid, blk, 0, e->stream, (const unsigned *)e->d_lat, dst, R, N, e->stride);
+        hipLaunchKernelGGL(unpack_bits<T>, bits_grid(R, N), blk, 0, e->stream, (const unsigned *)e->d_lat, dst, R, N, e->stride);
     } else {
         hipLaunchKernelGGL(unpack_hbm<T>, grid, blk, 0, e->stream, (const unsigned char *)e->d_lat, dst, R, N,
                            e->stride);
@@ -1113,12 +1123,7 @@ static int engine_unpack(gasp_engine *e, T *dst) {
 static int engine_get_grids_impl(gasp_engine *e, int *grids, int on_device) {
     const size_t bytes = (size_t)e->R * e->N * sizeof(int);
     if (on_device) return engine_unpack<int>(e, grids);
-    if (!e->d_tmp32 || e->tmp32_bytes < bytes) {
-        dfree(e->d_tmp32);
-        e->d_tmp32 = nullptr;
-        HIP_TRY(hipMalloc(&e->d_tmp32, bytes));
-        e->tmp32_bytes = bytes;
-    }
+    HIP_TRY(engine_scratch(e, bytes));
     int rc = engine_unpack<int>(e, e->d_tmp32);
     if (rc) return rc;
     HIP_TRY(hipMemcpyAsync(grids, e->d_tmp32, bytes, hipMemcpyDeviceToHost, e->stream));
@@ -1126,33 +1131,61 @@ static int engine_get_grids_impl(gasp_engine *e, int *grids, int on_device) {
 }
 
 // ------------------------------------------------------------ largest cluster
-// One workgroup per replica.  Labels and per-root sizes live in LDS when
-// 8*N bytes fit, else in a global workspace.  Lock-free union-find: every
-// site of the target spin starts as its own root; each site unites with its
-// right and lower neighbours (periodic) by hooking the larger root under the
-// smaller with atomicMin and retrying from the returned value when another
-// lane won the race; a final pass points every site at its root, sizes are
-// counted with atomics and the largest is reduced.
+// One workgroup per replica, on runs of equal spins.  The replica's spins come
+// from the native layout as bits (set: the target spin), and a row's runs are
+// then found with bit operations: only a run's first site carries a label.
+// Lock-free union-find over the runs: runs of neighbouring rows are united once
+// per stretch in which both rows are set (at its first column), and the two ends
+// of a row across the boundary, by hooking the larger root under the smaller with
+// atomicMin and retrying from the returned value when another lane won the race.
+// A last pass adds every run's length to its root's size, and the largest is
+// reduced.  What bounds it: the chains of dependent LDS reads in find() and the
+// bit tests per site.  1024 replicas of L = 64, half in each phase: 35 us,
+// 60 with a label and an addition per site on spins unpacked to bytes
+// (11 more).
+// Bits, labels and sizes (16 bits each: N < 65536) live in LDS when they fit,
+// else in a global workspace (32-bit sizes).
+static size_t cluster_bit_words(int N) { return ((size_t)N + 63) / 64 * 2; }
 template <bool USE_LDS>
-__global__ void __launch_bounds__(256) cluster_kernel(const int8_t *spins, int N, int L, int spin,
-                                                      int *work, float *out) {
+__global__ void __launch_bounds__(256) cluster_kernel(const void *lat, int layout, int stride, int N, int L, int spin,
+                                                      unsigned *work, float *out) {
     extern __shared__ __align__(16) unsigned char smem[];
     __shared__ int wmax[4];
-    const int r = blockIdx.x;
-    const int8_t *g = spins + (size_t)r * N;
-    int *lab, *cnt;
+    const int r = blockIdx.x, t = threadIdx.x, lane = t & 63;
+    const int nbw = (N + 63) / 64 * 2;
+    unsigned *bits, *cnt;
+    int *lab;
     if constexpr (USE_LDS) {
-        lab = (int *)smem;
-        cnt = lab + N;
+        bits = (unsigned *)smem;
+        lab = (int *)(bits + nbw);
+        cnt = (unsigned *)(lab + N);
     } else {
-        lab = work + (size_t)r * 2 * N;
-        cnt = lab + N;
+        bits = work + (size_t)r * (2 * (size_t)N + (size_t)nbw);
+        lab = (int *)(bits + nbw);
+        cnt = (unsigned *)(lab + N);
     }
-    const int t = threadIdx.x;
-    for (int i = t; i < N; i += blockDim.x) {
-        lab[i] = (g[i] == spin) ? i : -1;
-        cnt[i] = 0;
+    for (int x0 = t & ~63; x0 < N; x0 += 256) {
+        const int x = x0 + lane;
+        const bool up = x < N && spin_bits(lat, layout, stride, r, x, 1) != 0u;
+        const uint64_t m = wave_mask(x < N && (spin == 1 ? up : spin == -1 && !up));
+        if (lane < 2) bits[(x0 >> 5) + lane] = lane ? (unsigned)(m >> 32) : (unsigned)m;
     }
+    const int ncnt = USE_LDS ? (N + 1) / 2 : N;
+    for (int i = t; i < ncnt; i += 256) cnt[i] = 0u;
+    __syncthreads();
+    auto set = [&](int x) { return ((bits[x >> 5] >> (x & 31)) & 1u) != 0u; };
+    // the first site of x's run (row: the first site of its row)
+    auto run_start = [&](int x, int row) {
+        int w = x >> 5;
+        unsigned z = ~bits[w] & (0xffffffffu >> (31 - (x & 31)));
+        while (z == 0u && 32 * w > row) z = ~bits[--w];
+        const int s = z ? 32 * w + 32 - __clz((int)z) : 32 * w;
+        return max(s, row);
+    };
+    // first site of a run: labelled with itself
+    auto starts = [&](int x, int col) { return set(x) && (col == 0 || !set(x - 1)); };
+    for (int x = t; x < N; x += 256)
+        if (starts(x, x % L)) lab[x] = x;
     __syncthreads();
     auto find = [&](int x) {
         int y = lab[x];
@@ -1162,62 +1195,71 @@ __global__ void __launch_bounds__(256) cluster_kernel(const int8_t *spins, int N
         }
         return x;
     };
-    for (int i = t; i < N; i += blockDim.x) {
-        if (lab[i] < 0) continue;
-        const int row = i / L, col = i - row * L;
-        const int nb[2] = {row * L + (col == L - 1 ? 0 : col + 1), (row == L - 1 ? 0 : row + 1) * L + col};
-        for (int k = 0; k < 2; ++k) {
-            if (g[nb[k]] != spin) continue;
-            int a = find(i), b = find(nb[k]);
-            while (a != b) {
-                if (a < b) {
-                    const int tmp = a;
-                    a = b;
-                    b = tmp;
-                }
-                // a is the larger root: hook it under b
-                const int old = atomicMin(&lab[a], b);
-                if (old == a) break;
-                a = find(old);
-                b = find(b);
+    auto unite = [&](int a, int b) {
+        a = find(a);
+        b = find(b);
+        while (a != b) {
+            if (a < b) {
+                const int tmp = a;
+                a = b;
+                b = tmp;
             }
+            // a is the larger root: hook it under b
+            const int old = atomicMin(&lab[a], b);
+            if (old == a) break;
+            a = find(old);
+            b = find(b);
         }
+    };
+    for (int x = t; x < N; x += 256) {
+        if (!set(x)) continue;
+        const int col = x % L, row = x - col;
+        const int below = row + L == N ? 0 : row + L;  // the next row's first site
+        const int y = below + col;
+        if (set(y) && (col == 0 || !(set(x - 1) && set(y - 1)))) unite(run_start(x, row), run_start(y, below));
+        if (col == L - 1 && set(row)) unite(run_start(x, row), row);
     }
     __syncthreads();
-    for (int i = t; i < N; i += blockDim.x)
-        if (lab[i] >= 0) atomicAdd(&cnt[find(i)], 1);
+    for (int x = t; x < N; x += 256) {
+        const int col = x % L;
+        if (!starts(x, col)) continue;
+        const int end = x - col + L;  // the first site past the row
+        int w = x >> 5;
+        unsigned z = ~bits[w] & (0xffffffffu << (x & 31));
+        while (z == 0u && 32 * (w + 1) < end) z = ~bits[++w];
+        const int len = min(z ? 32 * w + __ffs((int)z) - 1 : end, end) - x;
+        const int root = find(x);
+        if constexpr (USE_LDS) atomicAdd(&cnt[root >> 1], (unsigned)len << (16 * (root & 1)));
+        else atomicAdd(&cnt[root], (unsigned)len);
+    }
     __syncthreads();
     int best = 0;
-    for (int i = t; i < N; i += blockDim.x) best = max(best, cnt[i]);
-    for (int off = 32; off >= 1; off >>= 1) best = max(best, __shfl_xor(best, off, 64));
-    if ((t & 63) == 0) wmax[t >> 6] = best;
-    __syncthreads();
-    if (t == 0) {
-        int m = 0;
-        for (int w = 0; w < (int)(blockDim.x >> 6); ++w) m = max(m, wmax[w]);
-        out[r] = (float)m;
+    for (int i = t; i < ncnt; i += 256) {
+        const unsigned c = cnt[i];
+        best = max(best, USE_LDS ? (int)max(c & 0xffffu, c >> 16) : (int)c);
     }
+    for (int off = 32; off >= 1; off >>= 1) best = max(best, __shfl_xor(best, off, 64));
+    if (lane == 0) wmax[t >> 6] = best;
+    __syncthreads();
+    if (t == 0) out[r] = (float)max(max(wmax[0], wmax[1]), max(wmax[2], wmax[3]));
 }
 
 static int engine_cluster(gasp_engine *e, int spin) {
-    const size_t n8 = (size_t)e->R * e->N;
-    if (!e->d_spins8) HIP_TRY(hipMalloc(&e->d_spins8, n8));
     if (!e->d_lclus) HIP_TRY(hipMalloc(&e->d_lclus, (size_t)e->R * sizeof(float)));
-    int rc = engine_unpack<int8_t>(e, e->d_spins8);
-    if (rc) return rc;
     DeviceInfo di = device_info();
-    const size_t lds = 8 * (size_t)e->N;
-    if (lds + 64 <= (di.ok ? di.lds_block : 65536)) {
+    const size_t N = (size_t)e->N, nbw = cluster_bit_words(e->N);
+    const size_t lds = 4 * (nbw + N + (N + 1) / 2);
+    if (N < 65536 && lds + 64 <= (di.ok ? di.lds_block : 65536)) {
         if (lds > 65536)
             HIP_TRY(hipFuncSetAttribute((const void *)cluster_kernel<true>,
                                         hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-        hipLaunchKernelGGL(cluster_kernel<true>, dim3(e->R), dim3(256), lds, e->stream, e->d_spins8, e->N, e->L,
-                           spin, (int *)nullptr, e->d_lclus);
+        hipLaunchKernelGGL(cluster_kernel<true>, dim3(e->R), dim3(256), lds, e->stream, (const void *)e->d_lat,
+                           e->layout, e->stride, e->N, e->L, spin, (unsigned *)nullptr, e->d_lclus);
     } else {
-        int *work = nullptr;
-        HIP_TRY(hipMallocAsync((void **)&work, (size_t)e->R * 2 * e->N * sizeof(int), e->stream));
-        hipLaunchKernelGGL(cluster_kernel<false>, dim3(e->R), dim3(256), 0, e->stream, e->d_spins8, e->N, e->L,
-                           spin, work, e->d_lclus);
+        unsigned *work = nullptr;
+        HIP_TRY(hipMallocAsync((void **)&work, (size_t)e->R * (2 * N + nbw) * sizeof(unsigned), e->stream));
+        hipLaunchKernelGGL(cluster_kernel<false>, dim3(e->R), dim3(256), 0, e->stream, (const void *)e->d_lat,
+                           e->layout, e->stride, e->N, e->L, spin, work, e->d_lclus);
         HIP_TRY(hipFreeAsync(work, e->stream));
     }
     HIP_TRY(hipGetLastError());
@@ -1289,20 +1331,12 @@ extern "C" int gasp_engine_get_gridstates(gasp_engine *e, uint8_t *host_out) {
     clear_error();
     if (!e || !host_out) return set_error(GASP_ERR_ARG, "gasp_engine_get_gridstates: NULL argument");
     const size_t nbytes = ((size_t)e->R * e->N + 7) / 8;
-    uint8_t *d = nullptr;
-    hipError_t he = hipMalloc(&d, nbytes);
-    if (he == hipSuccess) {
-        hipLaunchKernelGGL(pack_gridstates, dim3(2048), dim3(256), 0, e->stream, (const void *)e->d_lat, e->layout,
-                           e->stride, e->R, e->N, d, nbytes);
-        he = hipGetLastError();
-    }
-    if (he == hipSuccess) he = hipMemcpyAsync(host_out, d, nbytes, hipMemcpyDeviceToHost, e->stream);
-    if (he == hipSuccess) he = hipStreamSynchronize(e->stream);
-    dfree(d);
-    if (he != hipSuccess)
-        return set_error(he == hipErrorOutOfMemory ? GASP_ERR_NOMEM : GASP_ERR_HIP, "GPUassert: %s %s %d",
-                         hipGetErrorString(he), __FILE__, __LINE__);
-    return engine_collect_events(e);
+    if (hipError_t he = engine_scratch(e, nbytes)) return scratch_error(he);
+    uint8_t *d = (uint8_t *)e->d_tmp32;
+    launch_gridstates(e->d_lat, e->layout, e->stride, e->R, e->N, d, nbytes, e->stream);
+    HIP_TRY(hipGetLastError());
+    HIP_TRY(hipMemcpyAsync(host_out, d, nbytes, hipMemcpyDeviceToHost, e->stream));
+    return engine_sync(e);
 }
 
 extern "C" int gasp_engine_gather_grids(gasp_engine *e, const int *replicas, int n, int8_t *host_out) {
@@ -1314,25 +1348,16 @@ extern "C" int gasp_engine_gather_grids(gasp_engine *e, const int *replicas, int
         if (replicas[k] < 0 || replicas[k] >= e->R)
             return set_error(GASP_ERR_ARG, "gasp_engine_gather_grids: replica %d out of range [0, %d)", replicas[k],
                              e->R);
-    int *d_idx = nullptr;
-    int8_t *d_out = nullptr;
-    const size_t bytes = (size_t)n * e->N;
-    hipError_t he = hipMalloc(&d_idx, (size_t)n * sizeof(int));
-    if (he == hipSuccess) he = hipMalloc(&d_out, bytes);
-    if (he == hipSuccess) he = hipMemcpyAsync(d_idx, replicas, (size_t)n * sizeof(int), hipMemcpyHostToDevice, e->stream);
-    if (he == hipSuccess) {
-        hipLaunchKernelGGL(gather_spins8, dim3(1024), dim3(256), 0, e->stream, (const void *)e->d_lat, e->layout,
-                           e->stride, d_idx, n, e->N, d_out);
-        he = hipGetLastError();
-    }
-    if (he == hipSuccess) he = hipMemcpyAsync(host_out, d_out, bytes, hipMemcpyDeviceToHost, e->stream);
-    if (he == hipSuccess) he = hipStreamSynchronize(e->stream);
-    dfree(d_idx);
-    dfree(d_out);
-    if (he != hipSuccess)
-        return set_error(he == hipErrorOutOfMemory ? GASP_ERR_NOMEM : GASP_ERR_HIP, "GPUassert: %s %s %d",
-                         hipGetErrorString(he), __FILE__, __LINE__);
-    return engine_collect_events(e);
+    const size_t ibytes = align256((size_t)n * sizeof(int)), bytes = (size_t)n * e->N;
+    if (hipError_t he = engine_scratch(e, ibytes + bytes)) return scratch_error(he);
+    int *d_idx = e->d_tmp32;
+    int8_t *d_out = (int8_t *)e->d_tmp32 + ibytes;
+    HIP_TRY(hipMemcpyAsync(d_idx, replicas, (size_t)n * sizeof(int), hipMemcpyHostToDevice, e->stream));
+    hipLaunchKernelGGL(gather_spins8, bits_grid(n, e->N), dim3(256), 0, e->stream, (const void *)e->d_lat, e->layout,
+                       e->stride, d_idx, n, e->N, d_out);
+    HIP_TRY(hipGetLastError());
+    HIP_TRY(hipMemcpyAsync(host_out, d_out, bytes, hipMemcpyDeviceToHost, e->stream));
+    return engine_sync(e);
 }
 
 extern "C" int gasp_engine_sweep(gasp_engine *e, int nsweeps, int check, double dn_thr, double up_thr) {
@@ -1430,14 +1455,7 @@ extern "C" int gasp_engine_get_lattice_staging(gasp_engine *e, int *staging) {
 // compute_magnetisation_gpu) without an engine object.  The Philox key and
 // the attempt counter come from the RNG header in device memory and the
 // counter is advanced there by a kernel, so nothing is read back to the host
-// and consecutive calls continue one chain per replica.  A workspace holds,
-// at 256-byte aligned offsets: the 10 thresholds (0), 4 counters (128), the
-// magnetisation when the caller passes none (256: R floats) and the native
-// lattice.
-
-static size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
-
-
+// and consecutive calls continue one chain per replica.
 static int grids_check_args(int L, int R, int method, gasp_rng_state *d_state, const int *d_grids, int nsweeps) {
     if (L < 2 || L > 8192) return set_error(GASP_ERR_ARG, "Error: L must lie in [2, 8192]");
     if (R < 1) return set_error(GASP_ERR_ARG, "Error: ngrids must be positive");
@@ -1463,9 +1481,9 @@ static int sweep_grids_run(int L, int R, int method, gasp_rng_state *d_state, do
     const dim3 grid(1024), blk(256);
     const int lay = sh.win ? -1 : layout_of(method);  // sweep_window works on the caller's grids
     if (lay == 2)
-        hipLaunchKernelGGL(pack_multispin, grid, blk, 0, st, d_grids, (unsigned *)lat, R, N, sh.stride, 1);
+        hipLaunchKernelGGL(pack_multispin, dim3(4096), blk, 0, st, d_grids, (unsigned *)lat, R, N, sh.stride, 1);
     else if (lay == 1)
-        hipLaunchKernelGGL(pack_bits, grid, blk, 0, st, d_grids, (unsigned *)lat, R, N, sh.stride, 1);
+        hipLaunchKernelGGL(pack_bits, bits_grid(R, 32 * sh.stride), blk, 0, st, d_grids, (unsigned *)lat, R, N, sh.stride, 1);
     else if (lay == 0)
         hipLaunchKernelGGL(pack_hbm, grid, blk, 0, st, d_grids, (unsigned char *)lat, R, N, sh.stride, 1);
     HIP_TRY(hipGetLastError());
@@ -1500,9 +1518,9 @@ static int sweep_grids_run(int L, int R, int method, gasp_rng_state *d_state, do
         left -= nb;
     } while (left > 0);
     if (lay == 2)
-        hipLaunchKernelGGL(unpack_multispin<int>, grid, blk, 0, st, (const unsigned *)lat, d_grids, R, N, sh.stride);
+        hipLaunchKernelGGL(unpack_multispin<int>, dim3(4096), blk, 0, st, (const unsigned *)lat, d_grids, R, N, sh.stride);
     else if (lay == 1)
-        hipLaunchKernelGGL(unpack_bits<int>, grid, blk, 0, st, (const unsigned *)lat, d_grids, R, N, sh.stride);
+        hipLaunchKernelGGL(unpack_bits<int>, bits_grid(R, N), blk, 0, st, (const unsigned *)lat, d_grids, R, N, sh.stride);
     else if (lay == 0)
         hipLaunchKernelGGL(unpack_hbm<int>, grid, blk, 0, st, (const unsigned char *)lat, d_grids, R, N, sh.stride);
     HIP_TRY(hipGetLastError());
@@ -2147,8 +2165,7 @@ extern "C" void mc_driver_gpu(mc_gpu_grids_t grids, double beta, double h, int *
             if ((rc = engine_check_cv(e, e->d_lclus, check_mode, dn, up))) break;
         }
         if (do_grid && packed_out) {
-            hipLaunchKernelGGL(pack_gridstates, dim3(2048), dim3(256), 0, e->stream, (const void *)e->d_lat, e->layout,
-                               e->stride, R, e->N, d_bits, pbytes);
+            launch_gridstates(e->d_lat, e->layout, e->stride, R, e->N, d_bits, pbytes, e->stream);
             if (hipGetLastError() != hipSuccess ||
                 hipMemcpyAsync(h_bits, d_bits, pbytes, hipMemcpyDeviceToHost, e->stream) != hipSuccess) {
                 rc = set_error(GASP_ERR_HIP, "GPUassert: grid download");

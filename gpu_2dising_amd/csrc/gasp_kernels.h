@@ -1221,18 +1221,29 @@ __global__ void __launch_bounds__(64 * W) sweep_hbm_waves(SweepArgs a) {
 // Layout 2 in HBM: for group g (replicas 64g .. 64g+63) two dword planes of
 // `stride` dwords: plane 2g holds bit b < 32 of site s as bit b of dword s,
 // plane 2g + 1 the bits 32..63.  A split workgroup stages one plane.
-__global__ void pack_multispin(const int *__restrict__ src, unsigned *__restrict__ dst, int R, int N, int stride,
-                               int per) {
+// 16 replicas' loads are in flight at a time (16384 grids of L = 64, 268 MB read:
+// 142 us, 166 one after another).
+__global__ void __launch_bounds__(256) pack_multispin(const int *__restrict__ src, unsigned *__restrict__ dst, int R,
+                                                      int N, int stride, int per) {
     const int G = (R + 63) / 64;
     const size_t total = (size_t)G * N;
     for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < total; i += (size_t)gridDim.x * blockDim.x) {
         const int g = (int)(i / N), site = (int)(i - (size_t)g * N);
-        uint64_t w = 0;
         const int nb = min(64, R - 64 * g);
-        for (int b = 0; b < nb; ++b)
-            if (src[(size_t)((64 * g + b) / per) * N + site] == 1) w |= 1ull << b;
-        dst[(size_t)(2 * g) * stride + site] = (unsigned)w;
-        dst[(size_t)(2 * g + 1) * stride + site] = (unsigned)(w >> 32);
+        unsigned w[4] = {0u, 0u, 0u, 0u};
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            int v[16];
+#pragma unroll
+            for (int k = 0; k < 16; ++k) {
+                const int b = 16 * j + k, r = 64 * g + b;
+                v[k] = b < nb ? src[(size_t)(per == 1 ? r : r / per) * N + site] : 0;
+            }
+#pragma unroll
+            for (int k = 0; k < 16; ++k) w[j] |= (v[k] == 1 ? 1u : 0u) << k;
+        }
+        dst[(size_t)(2 * g) * stride + site] = w[0] | (w[1] << 16);
+        dst[(size_t)(2 * g + 1) * stride + site] = w[2] | (w[3] << 16);
     }
 }
 
@@ -1249,27 +1260,50 @@ __global__ void unpack_multispin(const unsigned *__restrict__ src, T *__restrict
     }
 }
 
-__global__ void pack_bits(const int *__restrict__ src, unsigned *__restrict__ dst, int R, int N, int stride,
-                          int per) {
-    const size_t total = (size_t)R * stride;
-    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < total; i += (size_t)gridDim.x * blockDim.x) {
-        const int r = (int)(i / stride), w = (int)(i - (size_t)r * stride);
-        unsigned v = 0;
-        for (int k = 0; k < 32; ++k) {
-            const int site = 32 * w + k;
-            if (site < N && src[(size_t)(r / per) * N + site] == 1) v |= 1u << k;
+// Bit lattice: blocks (x, y) take 1024 sites of the replicas y, y + gridDim.y, ...
+// (a block index per axis, no division per site).  A wave's 64 lanes read
+// neighbouring sites and a compare's lane mask is two words of the lattice:
+// 3001 grids of L = 75 in 18 us, 107 with a thread reading the 32 sites of
+// its word one by one.
+__host__ __device__ inline dim3 bits_grid(int R, int sites) {
+    const int x = (sites + 1023) / 1024, most = 8192 / x + 1;
+    return dim3((unsigned)x, (unsigned)(R < most ? R : most));
+}
+__global__ void __launch_bounds__(256) pack_bits(const int *__restrict__ src, unsigned *__restrict__ dst, int R, int N,
+                                                 int stride, int per) {
+    const int lane = threadIdx.x & 63;
+    const int x0 = (int)blockIdx.x * 1024 + (int)(threadIdx.x >> 6) * 256;  // the wave's first site
+    for (int r = blockIdx.y; r < R; r += gridDim.y) {
+        const int *s = src + (size_t)(r / per) * N;
+        int v[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int x = x0 + 64 * j + lane;
+            v[j] = x < N ? s[x] : 0;
         }
-        dst[i] = v;
+        unsigned w = 0u;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const uint64_t m = wave_mask(v[j] == 1);
+            if ((lane >> 1) == j) w = (lane & 1) ? (unsigned)(m >> 32) : (unsigned)m;
+        }
+        const int i = (x0 >> 5) + lane;  // words up to the stride: zero beyond N
+        if (lane < 8 && i < stride) dst[(size_t)r * stride + i] = w;
     }
 }
 
 template <typename T>
-__global__ void unpack_bits(const unsigned *__restrict__ src, T *__restrict__ dst, int R, int N, int stride) {
-    const size_t total = (size_t)R * N;
-    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < total; i += (size_t)gridDim.x * blockDim.x) {
-        const int r = (int)(i / N), site = (int)(i - (size_t)r * N);
-        const unsigned v = src[(size_t)r * stride + (site >> 5)];
-        dst[i] = ((v >> (site & 31)) & 1u) ? T(1) : T(-1);
+__global__ void __launch_bounds__(256) unpack_bits(const unsigned *__restrict__ src, T *__restrict__ dst, int R, int N,
+                                                   int stride) {
+    const int x0 = (int)blockIdx.x * 1024 + (int)threadIdx.x;
+    for (int r = blockIdx.y; r < R; r += gridDim.y) {
+        const unsigned *s = src + (size_t)r * stride;
+        T *d = dst + (size_t)r * N;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int x = x0 + 256 * j;
+            if (x < N) d[x] = ((s[x >> 5] >> (x & 31)) & 1u) ? T(1) : T(-1);
+        }
     }
 }
 
@@ -1357,49 +1391,96 @@ __global__ void __launch_bounds__(256) mt_draws_kernel(uint32_t *st, int R, uint
 // ------------------------------------------------------------ small kernels
 // (kernels rather than memset / host updates, so that they can be captured in
 // a graph and replayed)
+// Bits site .. site + n - 1 (n <= 32) of replica r, from any native layout.
+__device__ __forceinline__ unsigned spin_bits(const void *lat, int layout, int stride, int r, int site, int n) {
+    unsigned v = 0u;
+    if (layout == 1) {
+        const unsigned *w = (const unsigned *)lat + (size_t)r * stride + (site >> 5);
+        const int sh = site & 31;
+        v = w[0] >> sh;
+        if (sh + n > 32) v |= w[1] << (32 - sh);
+        return n < 32 ? v & ((1u << n) - 1u) : v;
+    }
+    if (layout == 2) {
+        const unsigned *w = (const unsigned *)lat + (size_t)(r >> 5) * stride + site;
+        for (int k = 0; k < n; ++k) v |= ((w[k] >> (r & 31)) & 1u) << k;
+    } else {
+        const unsigned char *c = (const unsigned char *)lat + (size_t)r * stride + site;
+        for (int k = 0; k < n; ++k) v |= (unsigned)(c[k] & 1) << k;
+    }
+    return v;
+}
+
 // The body of a gridstates.bin record (src/io.c:67-130): the R*N spins as one
 // bit stream, replica-major then site-major, bit k of byte b = spin 8b + k
-// (1 = up), padded with zero bits to whole bytes.  One thread per output byte.
-__global__ void pack_gridstates(const void *__restrict__ lat, int method, int stride, int R, int N,
-                                uint8_t *__restrict__ out, size_t nbytes) {
-    const size_t total = (size_t)R * N;
-    for (size_t b = (size_t)blockIdx.x * blockDim.x + threadIdx.x; b < nbytes; b += (size_t)gridDim.x * blockDim.x) {
-        unsigned v = 0;
-#pragma unroll
-        for (int k = 0; k < 8; ++k) {
-            const size_t i = 8 * b + k;
-            if (i >= total) break;
-            const int r = (int)(i / N), site = (int)(i - (size_t)r * N);
-            unsigned up;
-            if (method == 2) {
-                up = (((const unsigned *)lat)[(size_t)(r >> 5) * stride + site] >> (r & 31)) & 1u;
-            } else if (method == 1) {
-                up = (((const unsigned *)lat)[(size_t)r * stride + (site >> 5)] >> (site & 31)) & 1u;
-            } else {
-                up = ((const unsigned char *)lat)[(size_t)r * stride + site];
-            }
-            v |= up << k;
+// (1 = up), padded with zero bits to whole bytes.  A thread makes 32 bits, with
+// one division (2000 grids of L = 100: 5.4 us, 23 with one per bit).
+__global__ void __launch_bounds__(256) pack_gridstates(const void *__restrict__ lat, int layout, int stride, int R,
+                                                       int N, uint8_t *__restrict__ out, size_t nbytes) {
+    const size_t total = (size_t)R * N, nw = (nbytes + 3) / 4;
+    for (size_t w = (size_t)blockIdx.x * blockDim.x + threadIdx.x; w < nw; w += (size_t)gridDim.x * blockDim.x) {
+        const size_t i = 32 * w;
+        int r = total >> 32 ? (int)(i / N) : (int)((uint32_t)i / (uint32_t)N);
+        int site = (int)(i - (size_t)r * N);
+        unsigned v = 0u;
+        for (int k = 0; k < 32 && r < R; ++r, site = 0) {
+            const int n = min(32 - k, N - site);
+            v |= spin_bits(lat, layout, stride, r, site, n) << k;
+            k += n;
         }
-        out[b] = (uint8_t)v;
+        if (4 * w + 4 <= nbytes) {
+            *(uint32_t *)(out + 4 * w) = v;
+        } else {
+            for (size_t b = 4 * w; b < nbytes; ++b, v >>= 8) out[b] = (uint8_t)v;
+        }
     }
+}
+// The same from the multispin planes (layout 2) where N is a multiple of 64: a
+// wave turns 64 sites of a plane's 32 replicas, one coalesced read and a lane
+// mask per replica, into a 64-bit word for each (16384 grids of L = 64:
+// 19 us, 119 with every bit read by itself).
+__global__ void __launch_bounds__(256) pack_gridstates_planes(const unsigned *__restrict__ lat, int stride, int R,
+                                                              int N, uint64_t *__restrict__ out) {
+    const int lane = threadIdx.x & 63;
+    const unsigned chunks = (unsigned)N / 64, planes = ((unsigned)R + 31) / 32;
+    const unsigned waves = gridDim.x * (blockDim.x >> 6);
+    for (unsigned c = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6); c < (size_t)chunks * planes; c += waves) {
+        const unsigned p = c / chunks, k = c - p * chunks;
+        const unsigned v = lat[(size_t)p * stride + 64 * k + lane];
+        unsigned lo = 0u, hi = 0u;
+#pragma unroll
+        for (int b = 0; b < 32; ++b) {
+            const uint64_t m = wave_mask((v & (1u << b)) != 0u);
+            if (lane == b) {
+                lo = (unsigned)m;
+                hi = (unsigned)(m >> 32);
+            }
+        }
+        const unsigned r = 32 * p + lane;
+        if (lane < 32 && r < (unsigned)R) out[(size_t)r * chunks + k] = ((uint64_t)hi << 32) | lo;
+    }
+}
+inline void launch_gridstates(const void *lat, int layout, int stride, int R, int N, uint8_t *out, size_t nbytes,
+                              hipStream_t st) {
+    if (layout == 2 && N % 64 == 0)
+        hipLaunchKernelGGL(pack_gridstates_planes, dim3(2048), dim3(256), 0, st, (const unsigned *)lat, stride, R, N,
+                           (uint64_t *)out);
+    else
+        hipLaunchKernelGGL(pack_gridstates, dim3(2048), dim3(256), 0, st, lat, layout, stride, R, N, out, nbytes);
 }
 
 // Selected replicas idx[0..n) as int8 +-1 grids [n][N], from any native layout.
-__global__ void gather_spins8(const void *__restrict__ lat, int method, int stride, const int *__restrict__ idx,
-                              int n, int N, int8_t *__restrict__ out) {
-    const size_t total = (size_t)n * N;
-    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < total; i += (size_t)gridDim.x * blockDim.x) {
-        const int k = (int)(i / N), site = (int)(i - (size_t)k * N);
+__global__ void __launch_bounds__(256) gather_spins8(const void *__restrict__ lat, int layout, int stride,
+                                                     const int *__restrict__ idx, int n, int N,
+                                                     int8_t *__restrict__ out) {
+    const int x0 = (int)blockIdx.x * 1024 + (int)threadIdx.x;
+    for (int k = blockIdx.y; k < n; k += gridDim.y) {
         const int r = idx[k];
-        int up;
-        if (method == 2) {
-            up = (int)((((const unsigned *)lat)[(size_t)(r >> 5) * stride + site] >> (r & 31)) & 1u);
-        } else if (method == 1) {
-            up = (int)((((const unsigned *)lat)[(size_t)r * stride + (site >> 5)] >> (site & 31)) & 1u);
-        } else {
-            up = ((const unsigned char *)lat)[(size_t)r * stride + site];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int x = x0 + 256 * j;
+            if (x < N) out[(size_t)k * N + x] = spin_bits(lat, layout, stride, r, x, 1) ? (int8_t)1 : (int8_t)-1;
         }
-        out[i] = up ? (int8_t)1 : (int8_t)-1;
     }
 }
 
