@@ -77,12 +77,6 @@ __device__ __forceinline__ uint32_t spins_offset(uint32_t c, uint32_t up, uint32
     return x >> 25;
 }
 
-// A value that is the same in every lane, into scalar registers.
-__device__ __forceinline__ uint32_t uniform32(uint32_t x) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)x); }
-__device__ __forceinline__ uint64_t uniform64(uint64_t x) {
-    return ((uint64_t)uniform32((uint32_t)(x >> 32)) << 32) | uniform32((uint32_t)x);
-}
-
 template <int RNG, int W, bool POW2, int MODE, int IO>
 __global__ void __launch_bounds__(64 * W) sweep_window(SweepArgs a) {
     static_assert(W >= 1 && W <= 16 && (W & (W - 1)) == 0, "1 to 16 waves per replica");
