@@ -630,15 +630,16 @@ static int window_table_entries(int N, size_t lds, int per_cu) {
 // with the replicas as soon as the device is full, while the kernels that share
 // a workgroup between 8 to 64 replicas take as long for a few replicas as for
 // many, so it takes the smaller counts.  Method 2, 20 sweeps at L = 64: 256
-// replicas 0.21 ms against 2.11 on split words, 1024 0.37 against 2.14, 4096
-// 1.07 against 2.23, 8192 1.98 against 2.13, but 16384 3.70 against 3.20; 16384
-// at L = 48 2.07 against 2.10 and at L = 32 0.91 against 1.12; 8192 at L = 90
-// (10 sweeps) 2.13 against 2.15 and at L = 128 (5 sweeps) 2.38 against 2.41.
-// Method 1: 16384 at L = 64 (10 sweeps) 1.88 against 2.13, 65536 (5 sweeps)
-// 3.73 against 3.29, 16384 at L = 128 (2 sweeps) 2.10 against 1.68.  Method 0
-// is slower at every count: 16384 at L = 64 (10 sweeps) 1.90 against 3.01, 1024
-// at L = 256 (5 sweeps) 1.66 against 2.23.  An explicit shape, filter, staging
-// or table setting keeps the kernel that it is for.
+// replicas 0.21 ms against 2.10 on split words, 1024 0.29 against 2.19, 4096
+// 0.96 against 2.22, 8192 1.76 against 2.01, 10240 2.14 against 2.72, but 16384
+// 3.30 against 2.74 (52 replicas per CU where the lines cross; 10 sweeps of 16384 at
+// L = 48 0.97 against 0.93 and at L = 40 0.74 against 0.71, at L = 32 0.43 against
+// 0.47 but of 32768 0.84 against 0.69); 8192 at L = 90 (5 sweeps) 0.98 against
+// 1.02 and at L = 128 2.19 against 2.26.  Method 1: 16384 at L = 64 (10 sweeps)
+// 1.66 against 1.86, 65536 (5 sweeps) 3.27 against 3.14, 16384 at L = 128 (2 sweeps)
+// 1.97 against 1.46.  Method 0 is slower at every count: 16384 at L = 64 (10 sweeps)
+// 1.66 against 3.01, 256 at L = 256 (20 sweeps) 1.75 against 2.47.  An explicit
+// shape, filter, staging or table setting keeps the kernel that it is for.
 static void window_shape(int method, int L, int R, LaunchShape *sh) {
     if (method > 2 || g_tune_slots > 0 || g_tune_waves > 0 || g_tune_filter == 1 || g_tune_filter == 2 ||
         (g_tune_stage >= 1 && g_tune_stage <= 3) || g_tune_tables > 0)
@@ -646,7 +647,8 @@ static void window_shape(int method, int L, int R, LaunchShape *sh) {
     auto it = g_tuned.find(std::make_tuple(method, L, R));
     if (it != g_tuned.end() && !it->second.window) return;
     const long long ncu = sh->ncu;
-    if (!(method == 0 && L >= 32) && R > (L <= (method == 2 ? 48 : 64) ? 64 * ncu : 40 * ncu)) return;
+    const long long per_cu = L > 64 ? 40 : method == 2 && L > 32 ? 52 : 64;
+    if (!(method == 0 && L >= 32) && R > per_cu * ncu) return;
     DeviceInfo d = device_info();
     const size_t lds = d.ok ? d.lds_block : 65536;
     const int N = L * L;
@@ -663,9 +665,10 @@ static void window_shape(int method, int L, int R, LaunchShape *sh) {
     // Waves per replica: a window of 128 W attempts defers about 320 W / E of
     // them (E entries), and a CU is full from about 16 waves on.  Measured
     // fastest: 4 and 8 waves at L = 64 with 256 replicas (one workgroup per
-    // CU), 4 with 1024, 2 from 2048 on; 4 at L = 75 with 3001; 1 at L = 32 with
-    // 2048 and 2 with 256; 8 at L = 128 and 256 (sixteen never: 2.34 ms against
-    // 1.73 for 20 sweeps of 256 replicas at L = 256).
+    // CU), 4 with 1024, 2 from 2048 on; 2 at L = 48 with 8192; 4 at L = 75 and 90;
+    // 4 at L = 100 with 2000; 1 at L = 32 with 2048 and 2 with 256; 8 at L = 128 and
+    // 256 (sixteen never: 2.34 ms against 1.73 for 20 sweeps of 256 replicas at
+    // L = 256).
     const int E = M > 0 ? std::min(M, N) : N;
     int W = 1;
     for (int w = 2; w <= 8; w *= 2) {

@@ -32,16 +32,19 @@
 // table of keys with a power of two of entries (tbl_mask + 1; sites that share
 // one only add deferrals).
 //
-// What bounds it (L = 64, 16384 replicas, two waves each): the LDS pipe is busy
-// 70% of the cycles (23 instructions per wave and round, five and a half cycles
-// each, most of them bank conflicts of random sites) and VALU issue 66% (119
-// instructions per 128 attempts, against 124 in sweep_kernel with the mark
-// plane); a round defers 13% of its attempts.  With few workgroups per CU the
-// rounds are latency chains: Philox, the centre read, the mark, a barrier, the
-// entries, the threshold, a barrier.
-// Measured (100 sweeps of 256 replicas at L = 32 on two waves 0.62 ms, against
-// 4.54 on eighth words; 20 sweeps of 256 at L = 256, method 0, table, eight
-// waves 1.73 ms, against 2.45 on sweep_hbm_waves; other shapes at window_shape).
+// What bounds it (L = 64, 16384 replicas, two waves each): LDS instructions (23
+// per wave and round, seven cycles of the pipe for a read at random sites) and
+// instruction issue (119 vector and 62 scalar instructions per 128 attempts); a
+// round defers 13% of its attempts.  With few workgroups per CU the rounds are
+// latency chains: Philox, the centre read, the mark, a barrier, the entries, the
+// threshold, a barrier.  Either way waves wait for each other at the barriers, so
+// a wave's priority rises with how soon others need it: 0 while the words are
+// drawn (which the others' waits can hide), 2 up to the marks, 1 after the first
+// barrier and 3 from the flips to the second.
+// Measured (20 sweeps of 8192 replicas at L = 64 1.76 ms, 1.98 without the
+// priorities; 10 of 3001 at L = 75 0.48, 0.58; 100 of 256 at L = 32 on two waves
+// 0.62 ms, against 4.54 on eighth words; 20 of 256 at L = 256, method 0, table,
+// eight waves 1.75, against 2.45 on sweep_hbm_waves; other shapes at window_shape).
 //
 // IO 0: the engine's bit lattice (layout 1, uint32 [R][stride]); IO 1: the
 // caller's int32 +-1 grids [R][N], read and written in place.
@@ -188,7 +191,10 @@ __global__ void __launch_bounds__(64 * W) sweep_window(SweepArgs a) {
     uint32_t nxt = min(S, NP), ndef = 0u, left = kRounds;
     bool hold = false;
     uint32_t ahead = 0u;
+    // Wave priorities: lowest while the words are drawn, which can be done at any
+    // time, and highest before the barriers that other waves wait at.
     for (;;) {
+        __builtin_amdgcn_s_setprio(0);
         if (__builtin_amdgcn_inverse_ballot_w64(fresh)) {
             if constexpr (RNG == RNG_PHILOX) {
                 const uint64_t pair = P0 + q;
@@ -221,6 +227,7 @@ __global__ void __launch_bounds__(64 * W) sweep_window(SweepArgs a) {
             const uint64_t at = 6ull * (nxt + S) + 16ull * (uint32_t)tid;
             if (at < 6ull * (nxt + 2u * S) && at < 3ull * a.n_attempts) ahead = drw[at];
         }
+        __builtin_amdgcn_s_setprio(2);
         // the pair's keys (B's is one more); MODE 0 keeps the spin below them
         const uint32_t base = (left << kWinIdxBits) - 2u * (nxt - kWinSpan);
         const uint32_t kA = MODE == WIN_PACKED ? 4u * q + 2u * base : 2u * q + base;
@@ -241,6 +248,7 @@ __global__ void __launch_bounds__(64 * W) sweep_window(SweepArgs a) {
             oB = spins_offset(spin(sB.c), spin(sB.up), spin(sB.dn), spin(sB.lt), spin(sB.rt));
         }
         __syncthreads();
+        __builtin_amdgcn_s_setprio(1);
         uint64_t dA, dB;  // lanes with an earlier attempt in the stencil
         if constexpr (MODE == WIN_PACKED) {
             auto entry = [&](int x) { return lds_load32(kWinLat + (unsigned)x); };
@@ -268,6 +276,7 @@ __global__ void __launch_bounds__(64 * W) sweep_window(SweepArgs a) {
             fA &= wave_mask(may(oA));
             fB &= wave_mask(may(oB));
         }
+        __builtin_amdgcn_s_setprio(3);
         if (__builtin_amdgcn_inverse_ballot_w64(fA)) {
             if constexpr (MODE == WIN_PACKED) lds_xor32(kWinLat + (unsigned)sA.c, 1u);
             else lds_xor32(kWinLat + (((unsigned)sA.c >> 3) & ~3u), 1u << ((unsigned)sA.c & 31u));
