@@ -194,6 +194,10 @@ __global__ void __launch_bounds__(64 * W) sweep_sliced(SweepArgs a) {
         uint32_t blk = 0u;  // Philox block of the planes in w[]
         uint32_t w[4];
         const uint64_t A = a_begin + (uint64_t)l;
+        // A round ends when its slowest wave has decided all its replicas: of the
+        // waves that share a SIMD the one that is behind goes first (16384 replicas
+        // at L = 64, eight waves: 100 sweeps 4.29 -> 4.20 ms; the other way round 4.27).
+        __builtin_amdgcn_s_setprio(3);
         if (has) {
             w[0] = (uint32_t)A;
             w[1] = (uint32_t)(A >> 32);
@@ -222,6 +226,7 @@ __global__ void __launch_bounds__(64 * W) sweep_sliced(SweepArgs a) {
             // 1-4 of whole words, 3-10 of half words); they do not depend on
             // the lattice, so they are computed while its reads are in flight
             // (two independent chains side by side).
+            __builtin_amdgcn_s_setprio(2);
             uint32_t v1[4] = {(uint32_t)A, (uint32_t)(A >> 32), (uint32_t)g, kSlicedDomain + 1u};
             uint32_t v2[4] = {(uint32_t)A, (uint32_t)(A >> 32), (uint32_t)g, kSlicedDomain + 2u};
             philox4x32_10x2(v1, v2, k0, k1);
@@ -309,6 +314,7 @@ __global__ void __launch_bounds__(64 * W) sweep_sliced(SweepArgs a) {
 #pragma unroll
             for (int d = 1; d < Q; ++d) pend |= und[d];
             blk = 2u;
+            __builtin_amdgcn_s_setprio(1);
             while (wave_mask(pend != 0u) != 0ull && p < 32) {
                 uint32_t va[4] = {(uint32_t)A, (uint32_t)(A >> 32), (uint32_t)g, kSlicedDomain + blk + 1u};
                 uint32_t vb[4] = {(uint32_t)A, (uint32_t)(A >> 32), (uint32_t)g, kSlicedDomain + blk + 2u};
@@ -335,6 +341,7 @@ __global__ void __launch_bounds__(64 * W) sweep_sliced(SweepArgs a) {
 #pragma unroll
             for (int d = 0; d < Q; ++d) flip[d] = acc[d];
         }
+        __builtin_amdgcn_s_setprio(0);
         if (had_prev) lds_ptr32(kSlLat + prev_pos + 8u + 4u * (par ^ 1u))[0] = ~0u;
         __syncthreads();
         bool deferred = false;
