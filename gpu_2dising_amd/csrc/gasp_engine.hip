@@ -1010,20 +1010,28 @@ static int launch_sweep(gasp_engine *e, uint64_t n_attempts, const uint32_t *dra
     memcpy(a.thr, e->thr, sizeof a.thr);
     a.mag = e->d_mag;
     a.fate = e->d_fate;
-    a.counts = e->d_counts;
+    a.counts = e->win ? nullptr : e->d_counts;  // one replica per workgroup: counted after the sweep
     a.check = check;
     a.freeze = e->freeze;
     a.tbl_mask = (unsigned)(e->tbl - 1);
     a.dn_thr = dn;
     a.up_thr = up;
     SweepFn fn = engine_fn(e);
-    if (check != CHECK_NONE) {
+    if (check != CHECK_NONE && !e->win) {
         hipLaunchKernelGGL(zero_ints, dim3(1), dim3(64), 0, e->stream, e->d_counts, 4);
         HIP_TRY(hipGetLastError());
     }
+    auto count = [&]() -> int {
+        if (check == CHECK_NONE || !e->win) return GASP_OK;
+        hipLaunchKernelGGL(count_checks, dim3(1), dim3(1024), 0, e->stream, (const float *)e->d_mag,
+                           (const int *)e->d_fate, e->R, check, up, e->d_counts);
+        HIP_TRY(hipGetLastError());
+        return GASP_OK;
+    };
     if (capture) {
         hipLaunchKernelGGL(fn, dim3(e->nblocks), dim3(e->block), e->lds, e->stream, a);
         HIP_TRY(hipGetLastError());
+        if (const int rc = count()) return rc;
         hipLaunchKernelGGL(advance_counter, dim3(1), dim3(64), 0, e->stream, (RngHeader *)e->d_rng, e->R,
                            n_attempts);
         HIP_TRY(hipGetLastError());
@@ -1038,6 +1046,7 @@ static int launch_sweep(gasp_engine *e, uint64_t n_attempts, const uint32_t *dra
     HIP_TRY(hipEventRecord(ev1, e->stream));
     e->ev_pending.push_back(ev0);
     e->ev_pending.push_back(ev1);
+    if (const int rc = count()) return rc;
     e->launches++;
     e->rng.attempts += n_attempts;
     return GASP_OK;
@@ -1096,7 +1105,7 @@ static int engine_set_grids_impl(gasp_engine *e, const int *grids, int on_device
     const int N = e->N, R = e->R, per = R / ninputs;
     const dim3 grid(1024), blk(256);
     if (e->layout == 2) {
-        hipLaunchKernelGGL(pack_multispin, dim3(4096), blk, 0, e->stream, src, (unsigned *)e->d_lat, R, N, e->stride, per);
+        hipLaunchKernelGGL(pack_multispin, blocks_for((size_t)(R + 63) / 64 * N, 4096), blk, 0, e->stream, src, (unsigned *)e->d_lat, R, N, e->stride, per);
     } else if (e->layout == 1) {
         hipLaunchKernelGGL(pack_bits, bits_grid(R, 32 * e->stride), blk, 0, e->stream, src, (unsigned *)e->d_lat, R, N, e->stride, per);
     } else {
@@ -1111,7 +1120,7 @@ static int engine_unpack(gasp_engine *e, T *dst) {
     const int N = e->N, R = e->R;
     const dim3 grid(1024), blk(256);
     if (e->layout == 2) {
-        hipLaunchKernelGGL(unpack_multispin<T>, dim3(4096), blk, 0, e->stream, (const unsigned *)e->d_lat, dst, R, N,
+        hipLaunchKernelGGL(unpack_multispin<T>, blocks_for((size_t)(R + 63) / 64 * N, 4096), blk, 0, e->stream, (const unsigned *)e->d_lat, dst, R, N,
                            e->stride);
     } else if (e->layout == 1) {
         hipLaunchKernelGGL(unpack_bits<T>, bits_grid(R, N), blk, 0, e->stream, (const unsigned *)e->d_lat, dst, R, N, e->stride);
@@ -1484,7 +1493,7 @@ static int sweep_grids_run(int L, int R, int method, gasp_rng_state *d_state, do
     const dim3 grid(1024), blk(256);
     const int lay = sh.win ? -1 : layout_of(method);  // sweep_window works on the caller's grids
     if (lay == 2)
-        hipLaunchKernelGGL(pack_multispin, dim3(4096), blk, 0, st, d_grids, (unsigned *)lat, R, N, sh.stride, 1);
+        hipLaunchKernelGGL(pack_multispin, blocks_for((size_t)(R + 63) / 64 * N, 4096), blk, 0, st, d_grids, (unsigned *)lat, R, N, sh.stride, 1);
     else if (lay == 1)
         hipLaunchKernelGGL(pack_bits, bits_grid(R, 32 * sh.stride), blk, 0, st, d_grids, (unsigned *)lat, R, N, sh.stride, 1);
     else if (lay == 0)
@@ -1521,7 +1530,7 @@ static int sweep_grids_run(int L, int R, int method, gasp_rng_state *d_state, do
         left -= nb;
     } while (left > 0);
     if (lay == 2)
-        hipLaunchKernelGGL(unpack_multispin<int>, dim3(4096), blk, 0, st, (const unsigned *)lat, d_grids, R, N, sh.stride);
+        hipLaunchKernelGGL(unpack_multispin<int>, blocks_for((size_t)(R + 63) / 64 * N, 4096), blk, 0, st, (const unsigned *)lat, d_grids, R, N, sh.stride);
     else if (lay == 1)
         hipLaunchKernelGGL(unpack_bits<int>, bits_grid(R, N), blk, 0, st, (const unsigned *)lat, d_grids, R, N, sh.stride);
     else if (lay == 0)

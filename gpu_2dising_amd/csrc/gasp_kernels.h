@@ -504,6 +504,7 @@ __device__ __forceinline__ void finish_replica(const SweepArgs &a, bool own, int
             is_b = (f == 1);
         }
     }
+    if (!a.counts) return;  // counted afterwards (count_checks)
     if (a.check == CHECK_COUNT) {
         const uint64_t b = wave_mask(gt_up);
         if ((threadIdx.x & 63) == 0 && b) atomicAdd(&a.counts[0], (int)__popcll(b));
@@ -1243,6 +1244,13 @@ __global__ void __launch_bounds__(64 * W) sweep_hbm_waves(SweepArgs a) {
 }
 
 // ------------------------------------------------------------ layout kernels
+// Blocks of 256 threads for a grid-stride loop over `total` items: no more than
+// have one (an empty block still has to be launched).
+inline dim3 blocks_for(size_t total, size_t most) {
+    const size_t b = (total + 255) / 256;
+    return dim3((unsigned)(b < most ? b : most));
+}
+
 // int32 +-1 grids [R][N] <-> native layouts.  1-D grid-stride loops over
 // (replica or group, element) so that any R fits the launch limits.
 // `per` consecutive replicas share one source grid (1: one grid per replica;
@@ -1432,9 +1440,11 @@ __device__ __forceinline__ unsigned spin_bits(const void *lat, int layout, int s
     }
     if (layout == 2) {
         const unsigned *w = (const unsigned *)lat + (size_t)(r >> 5) * stride + site;
+#pragma unroll 8
         for (int k = 0; k < n; ++k) v |= ((w[k] >> (r & 31)) & 1u) << k;
     } else {
         const unsigned char *c = (const unsigned char *)lat + (size_t)r * stride + site;
+#pragma unroll 8
         for (int k = 0; k < n; ++k) v |= (unsigned)(c[k] & 1) << k;
     }
     return v;
@@ -1442,22 +1452,28 @@ __device__ __forceinline__ unsigned spin_bits(const void *lat, int layout, int s
 
 // The body of a gridstates.bin record (src/io.c:67-130): the R*N spins as one
 // bit stream, replica-major then site-major, bit k of byte b = spin 8b + k
-// (1 = up), padded with zero bits to whole bytes.  A thread makes 32 bits, with
-// one division (2000 grids of L = 100: 5.4 us, 23 with one per bit).
+// (1 = up), padded with zero bits to whole bytes.  A thread makes BITS of them with
+// one division: 32 from the bit lattice (2000 grids of L = 100: 5.4 us, 23 with a
+// division per bit), 8 from bytes and planes, where a wave then reads neighbouring
+// sites (32 from planes: 12000 grids of L = 140 in 0.94 ms against 0.066).
+template <int BITS>
 __global__ void __launch_bounds__(256) pack_gridstates(const void *__restrict__ lat, int layout, int stride, int R,
                                                        int N, uint8_t *__restrict__ out, size_t nbytes) {
-    const size_t total = (size_t)R * N, nw = (nbytes + 3) / 4;
+    constexpr int kBytes = BITS / 8;
+    const size_t total = (size_t)R * N, nw = (nbytes + kBytes - 1) / kBytes;
     for (size_t w = (size_t)blockIdx.x * blockDim.x + threadIdx.x; w < nw; w += (size_t)gridDim.x * blockDim.x) {
-        const size_t i = 32 * w;
+        const size_t i = BITS * w;
         int r = total >> 32 ? (int)(i / N) : (int)((uint32_t)i / (uint32_t)N);
         int site = (int)(i - (size_t)r * N);
         unsigned v = 0u;
-        for (int k = 0; k < 32 && r < R; ++r, site = 0) {
-            const int n = min(32 - k, N - site);
+        for (int k = 0; k < BITS && r < R; ++r, site = 0) {
+            const int n = min(BITS - k, N - site);
             v |= spin_bits(lat, layout, stride, r, site, n) << k;
             k += n;
         }
-        if (4 * w + 4 <= nbytes) {
+        if constexpr (BITS == 8) {
+            out[w] = (uint8_t)v;
+        } else if (4 * w + 4 <= nbytes) {
             *(uint32_t *)(out + 4 * w) = v;
         } else {
             for (size_t b = 4 * w; b < nbytes; ++b, v >>= 8) out[b] = (uint8_t)v;
@@ -1492,10 +1508,14 @@ __global__ void __launch_bounds__(256) pack_gridstates_planes(const unsigned *__
 inline void launch_gridstates(const void *lat, int layout, int stride, int R, int N, uint8_t *out, size_t nbytes,
                               hipStream_t st) {
     if (layout == 2 && N % 64 == 0)
-        hipLaunchKernelGGL(pack_gridstates_planes, dim3(2048), dim3(256), 0, st, (const unsigned *)lat, stride, R, N,
-                           (uint64_t *)out);
+        hipLaunchKernelGGL(pack_gridstates_planes, blocks_for((size_t)(R + 31) / 32 * N, 2048), dim3(256), 0, st,
+                           (const unsigned *)lat, stride, R, N, (uint64_t *)out);
+    else if (layout == 1)
+        hipLaunchKernelGGL(pack_gridstates<32>, blocks_for((nbytes + 3) / 4, 2048), dim3(256), 0, st, lat, layout, stride,
+                           R, N, out, nbytes);
     else
-        hipLaunchKernelGGL(pack_gridstates, dim3(2048), dim3(256), 0, st, lat, layout, stride, R, N, out, nbytes);
+        hipLaunchKernelGGL(pack_gridstates<8>, blocks_for(nbytes, 8192), dim3(256), 0, st, lat, layout, stride, R, N, out,
+                           nbytes);
 }
 
 // Selected replicas idx[0..n) as int8 +-1 grids [n][N], from any native layout.
@@ -1516,6 +1536,42 @@ __global__ void __launch_bounds__(256) gather_spins8(const void *__restrict__ la
 __global__ void zero_ints(int *p, int n) {
     if ((int)threadIdx.x < n) p[threadIdx.x] = 0;
 }
+// The threshold check's counts from the magnetisations and fates, for sweeps of
+// one replica per workgroup: there each replica's atomic addition to the one
+// count would follow the others' (12000 replicas of L = 20, one sweep: 0.12 ms of
+// 0.15, against 4 us here).  One workgroup; writes all four counts.
+__global__ void __launch_bounds__(1024) count_checks(const float *__restrict__ mag, const int *__restrict__ fate, int R,
+                                                     int check, double up_thr, int *__restrict__ counts) {
+    __shared__ int sum[3];
+    const int t = threadIdx.x;
+    if (t < 3) sum[t] = 0;
+    __syncthreads();
+    int up = 0, is_a = 0, is_b = 0;
+    for (int r = t; r < R; r += 1024) {
+        const float m = mag[r];
+        if (check == CHECK_COUNT) {
+            up += (double)m > up_thr ? 1 : 0;
+        } else if (m == m) {  // NaN: the sweep refused its RNG header
+            const int f = fate[r];
+            is_a += f == 0 ? 1 : 0;
+            is_b += f == 1 ? 1 : 0;
+        }
+    }
+#pragma unroll
+    for (int off = 32; off >= 1; off >>= 1) {
+        up += __shfl_xor(up, off, 64);
+        is_a += __shfl_xor(is_a, off, 64);
+        is_b += __shfl_xor(is_b, off, 64);
+    }
+    if ((t & 63) == 0) {
+        atomicAdd(&sum[0], up);
+        atomicAdd(&sum[1], is_a);
+        atomicAdd(&sum[2], is_b);
+    }
+    __syncthreads();
+    if (t < 4) counts[t] = t < 3 ? sum[t] : 0;
+}
+
 // Advances the attempt counter of a device RNG header by n, if the header
 // is one the sweep kernels accept for R replicas (they did not sweep otherwise).
 __global__ void advance_counter(RngHeader *hdr, int R, uint64_t n) {
