@@ -7,6 +7,9 @@
 //   global average pool -> fc1 32->64 + ReLU -> fc2 64->1 -> sigmoid = pB
 // trained with binary cross-entropy against shooting labels.
 //
+// L <= 64: the layers joined in LDS, gasp_cnn_stream.h, with conv1, the head, the
+// reductions' order and Adam as here.  L >= 128: a kernel per layer, below.
+//
 // Storage: activations NHWC bfloat16 [n][L][L][32]; conv2..4 weights as MFMA
 // fragments (bfloat16); conv1 weights and the MLP in float32.  Parameters are
 // one float32 vector (30241 entries) in the order
