@@ -675,6 +675,11 @@ struct gasp_cnn {
             return set_error(GASP_ERR_HIP, "GPUassert: %s %s %d", hipGetErrorString(q_), __FILE__, __LINE__); \
     } while (0)
 
+// Inference, L <= 64: four images a workgroup (and 64 / L side by side) per piece
+// of the upload, the next piece beside the kernels on this one.  4096 grids of
+// L = 64: 1205 us in one piece, 945 in four.
+static int upload_piece(const gasp_cnn *c) { return 4 * c->ncu * (64 / c->L); }
+
 static void cfree(void *p) {
     if (p) (void)hipFree(p);
 }
@@ -755,9 +760,11 @@ extern "C" int gasp_cnn_create(int L, int max_batch, gasp_cnn **out) {
     if (e == hipSuccess) e = hipGetDevice(&dev);
     if (e == hipSuccess) e = hipDeviceGetAttribute(&c->ncu, hipDeviceAttributeMultiprocessorCount, dev);
     if (c->stream) {
-        if (e == hipSuccess) e = hipStreamCreateWithFlags(&c->cst, hipStreamNonBlocking);
-        if (e == hipSuccess) e = hipEventCreateWithFlags(&c->up, hipEventDisableTiming);
-        if (e == hipSuccess) e = hipEventCreateWithFlags(&c->done, hipEventDisableTiming);
+        if (max_batch > upload_piece(c)) {
+            if (e == hipSuccess) e = hipStreamCreateWithFlags(&c->cst, hipStreamNonBlocking);
+            if (e == hipSuccess) e = hipEventCreateWithFlags(&c->up, hipEventDisableTiming);
+            if (e == hipSuccess) e = hipEventCreateWithFlags(&c->done, hipEventDisableTiming);
+        }
         A((void **)&c->tab, 512 * C * 2);
         A((void **)&c->m4, n * N * 4);
         A((void **)&c->code, n * N * 2);
@@ -983,10 +990,7 @@ extern "C" int gasp_cnn_predict(gasp_cnn *c, const int8_t *spins, int n, float *
     gasp::clear_error();
     if (!c || !spins || !pB || n < 0) return set_error(GASP_ERR_ARG, "gasp_cnn_predict: bad argument");
     if (!c->weights_ready) return set_error(GASP_ERR_ARG, "gasp_cnn_predict: parameters not set");
-    // Four images a workgroup (and 64 / L side by side) per piece: the next piece
-    // is uploaded while the kernels run on this one.  4096 grids of L = 64: 1205 us
-    // in one piece, 945 in four.
-    const int piece = c->stream ? 4 * c->ncu * (64 / c->L) : c->nmax;
+    const int piece = c->stream ? upload_piece(c) : c->nmax;
     for (int i0 = 0; i0 < n; i0 += c->nmax) {
         const int nb = std::min(c->nmax, n - i0);
         if (c->stream && nb > piece) {
