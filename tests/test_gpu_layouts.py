@@ -64,3 +64,23 @@ def test_largest_cluster_workspace(gpu, engine_lib, oracle, L):
             ref = [lib.orc_largest_cluster(L, g[r].reshape(-1), spin) for r in range(R)]
             assert np.array_equal(e.largest_cluster(spin), np.array(ref, dtype=np.float32)), spin
     rng.free()
+
+
+@pytest.mark.parametrize("R", [1, 64, 1023, 1025, 3000])
+def test_counts_of_the_check(gpu, engine_lib, R):
+    """The check's counts, summed by one workgroup of 1024 lanes, against the magnetisations and fates."""
+    G = engine_lib
+    L = 8
+    print(f"[counts] R={R}", flush=True)
+    rng = G.RngState(R, 3)
+    with G.Engine(L, R, 2, rng, 0.3, 0.0) as e:
+        e.set_grids(_patterns(R, L, R))
+        e.sweep(1, G.CHECK_COUNT, -0.2, 0.2)
+        m = e.magnetisation().astype(np.float64)
+        assert list(e.counts()) == [int((m > 0.2).sum()), 0, 0, 0][:len(e.counts())]
+        e.set_fates(np.full(R, -1, dtype=np.int32))
+        for _ in range(2):
+            e.sweep(1, G.CHECK_FATES, -0.2, 0.2)
+            f = e.fates()
+            assert list(e.counts()) == [0, int((f == 0).sum()), int((f == 1).sum()), 0][:len(e.counts())]
+    rng.free()
