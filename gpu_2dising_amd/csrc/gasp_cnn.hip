@@ -8,7 +8,8 @@
 // trained with binary cross-entropy against shooting labels.
 //
 // L <= 64: the layers joined in LDS, gasp_cnn_stream.h, with conv1, the head, the
-// reductions' order and Adam as here.  L >= 128: a kernel per layer, below.
+// reductions' order and Adam as here.  L >= 128, and batches of L <= 64 with other
+// values than +-1: a kernel per layer, below.
 //
 // Storage: activations NHWC bfloat16 [n][L][L][32]; conv2..4 weights as MFMA
 // fragments (bfloat16); conv1 weights and the MLP in float32.  Parameters are
@@ -636,6 +637,20 @@ __global__ void gather_batch(const int8_t *__restrict__ data, const float *__res
 
 #include "gasp_cnn_stream.h"
 
+namespace cnn {
+
+// Whether `words` times 16 bytes hold any other value than +-1.
+__global__ void __launch_bounds__(256) find_odd(const uint4 *__restrict__ s, size_t words, int *__restrict__ odd) {
+    uint32_t bad = 0u;
+    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < words; i += (size_t)gridDim.x * blockDim.x) {
+        const uint4 v = s[i];
+        bad |= not_spins(v.x) | not_spins(v.y) | not_spins(v.z) | not_spins(v.w);
+    }
+    if (bad) *odd = 1;
+}
+
+}  // namespace cnn
+
 using namespace cnn;
 
 // =================================================================== host side
@@ -652,6 +667,8 @@ struct gasp_cnn {
     uint16_t *dz0 = nullptr, *dz1 = nullptr;
     float *part = nullptr, *part1 = nullptr, *part_head = nullptr;
     float *red = nullptr;  // chunk sums of the two-level reductions
+    int *odd = nullptr;    // set where a streamed batch holds other values than +-1; the word before loss
+    bool data_odd = false;  // the stored data do
     bool stream = false;   // L <= 64: whole images through a workgroup (gasp_cnn_stream.h)
     int ncu = 256;
     uint16_t *tab = nullptr;            // conv1's table
@@ -691,7 +708,7 @@ extern "C" int gasp_cnn_destroy(gasp_cnn *c) {
     if (c->st) (void)hipStreamSynchronize(c->st);
     if (c->cst) (void)hipStreamSynchronize(c->cst);
     for (void *q : {(void *)c->p, (void *)c->g, (void *)c->m, (void *)c->v, (void *)c->w1r, (void *)c->wf,
-                    (void *)c->wb, (void *)c->s, (void *)c->y, (void *)c->pb, (void *)c->loss, (void *)c->dg,
+                    (void *)c->wb, (void *)c->s, (void *)c->y, (void *)c->pb, (void *)c->odd, (void *)c->dg,
                     (void *)c->a[1], (void *)c->a[2], (void *)c->a[3], (void *)c->a[4], (void *)c->dz0,
                     (void *)c->dz1, (void *)c->part, (void *)c->part1, (void *)c->part_head,
                     (void *)c->red, (void *)c->data, (void *)c->data_y, (void *)c->data_loss, (void *)c->order, (void *)c->tab, (void *)c->m4, (void *)c->code,
@@ -722,6 +739,30 @@ static hipError_t net_attributes() {
     return hipSuccess;
 }
 
+static size_t red_bytes(size_t n, int L) {
+    const size_t q = (size_t)kRedChunk;
+    return std::max({(n * 4 + q - 1) / q * kWgRow, (n * L + q - 1) / q * 320, (n + q - 1) / q * HEAD_N}) * 4;
+}
+
+// What the separate kernels need beyond the streamed ones' buffers, made when a
+// batch first needs them: a1 and the chunk sums (a4 lies in dz1 until conv4's
+// backward, which writes there, has read it; the partial gradients in parts[2]).
+static int layer_buffers(gasp_cnn *c) {
+    const size_t n = (size_t)c->nmax;
+    hipError_t e = hipSuccess;
+    if (!c->a[1]) e = hipMalloc((void **)&c->a[1], n * c->N * C * 2);
+    if (e == hipSuccess && !c->red) e = hipMalloc((void **)&c->red, red_bytes(n, c->L));
+    if (e != hipSuccess)
+        return set_error(e == hipErrorOutOfMemory ? GASP_ERR_NOMEM : GASP_ERR_HIP, "gasp_cnn: %s", hipGetErrorString(e));
+    return GASP_OK;
+}
+// A streamed batch has reported other values than +-1: the report is taken back,
+// and the batch goes through the separate kernels.
+static int to_layers(gasp_cnn *c) {
+    CTRY(hipMemsetAsync(c->odd, 0, 4, c->st));
+    return layer_buffers(c);
+}
+
 extern "C" int gasp_cnn_create(int L, int max_batch, gasp_cnn **out) {
     gasp::clear_error();
     if (!out) return set_error(GASP_ERR_ARG, "gasp_cnn_create: NULL output");
@@ -748,7 +789,8 @@ extern "C" int gasp_cnn_create(int L, int max_batch, gasp_cnn **out) {
     A((void **)&c->s, n * N);
     A((void **)&c->y, n * 4);
     A((void **)&c->pb, n * 4);
-    A((void **)&c->loss, n * 4);
+    A((void **)&c->odd, (n + 1) * 4);
+    if (c->odd) c->loss = (float *)c->odd + 1;
     A((void **)&c->dg, n * C * 4);
     A((void **)&c->a[2], n * N * C * 2);
     A((void **)&c->a[3], n * N * C * 2);
@@ -777,9 +819,7 @@ extern "C" int gasp_cnn_create(int L, int max_batch, gasp_cnn **out) {
         A((void **)&c->a[4], n * N * C * 2);
         A((void **)&c->part, n * 4 * kWgRow * 4);
         A((void **)&c->part1, n * (size_t)L * 320 * 4);
-        const size_t q = (size_t)kRedChunk;
-        const size_t r = std::max({(n * 4 + q - 1) / q * kWgRow, (n * L + q - 1) / q * 320, (n + q - 1) / q * HEAD_N});
-        A((void **)&c->red, r * 4);
+        A((void **)&c->red, red_bytes(n, L));
     }
     if (e == hipSuccess) e = hipStreamSynchronize(c->st);
     if (e != hipSuccess) {
@@ -862,9 +902,9 @@ static int infer_stream(gasp_cnn *c, const int8_t *s, int n, float *pb) {
     const NetShape g = net_shape(c, n);
     hipLaunchKernelGGL((net_fwd<false, LG>), dim3(std::min(g.units, c->ncu)), dim3(kFwdThreads), kFwdLds, c->st, s, c->wf, c->p,
                        c->w1r, (uint16_t *)nullptr, (uint16_t *)nullptr, (uint16_t *)nullptr, (uint32_t *)nullptr, c->pool,
-                       (uint16_t *)nullptr, (uint16_t *)nullptr, g);
+                       (uint16_t *)nullptr, (uint16_t *)nullptr, c->odd, g);
     hipLaunchKernelGGL((net_head<false, LG>), dim3(n), dim3(64), 0, c->st, c->pool, c->p, (const float *)nullptr, pb, c->loss,
-                       c->part_head, c->dg, g, 0.0f);
+                       c->part_head, c->dg, c->odd, g, 0.0f);
     CTRY(hipGetLastError());
     return GASP_OK;
 }
@@ -883,13 +923,13 @@ static int forward_stream(gasp_cnn *c, int n, const float *d_labels) {
     // dz1, free until net_back<3>) and `head` pools it.
     uint16_t *a4 = g.nb > 1 ? c->dz1 : nullptr;
     hipLaunchKernelGGL((net_fwd<true, LG>), grid, dim3(kFwdThreads), kFwdLds, c->st, c->s, c->wf, c->p, c->w1r, c->a[2],
-                       c->a[3], a4, c->m4, c->pool, c->tab, c->code, g);
+                       c->a[3], a4, c->m4, c->pool, c->tab, c->code, c->odd, g);
     if (a4)
         hipLaunchKernelGGL(head, dim3(n), dim3(256), 0, c->st, a4, c->p, d_labels, c->pb, c->loss, c->part_head, c->dg, n,
                            c->L, 1.0f / (float)n);
     else
         hipLaunchKernelGGL((net_head<true, LG>), dim3(n), dim3(64), 0, c->st, c->pool, c->p, d_labels, c->pb, c->loss,
-                           c->part_head, c->dg, g, 1.0f / (float)n);
+                           c->part_head, c->dg, c->odd, g, 1.0f / (float)n);
     CTRY(hipGetLastError());
     return GASP_OK;
 }
@@ -925,9 +965,10 @@ static int backward_stream(gasp_cnn *c, int n, const AdamArgs *ad) {
     return c->L == 64 ? backward_stream<6>(c, n, ad) : c->L == 32 ? backward_stream<5>(c, n, ad) : backward_stream<4>(c, n, ad);
 }
 
-// forward of n <= nmax grids already in c->s
-static int forward(gasp_cnn *c, int n, const float *d_labels) {
-    if (c->stream)
+// forward of n <= nmax grids already in c->s, by the streamed kernels or (L >= 128, or
+// after layer_buffers) by the separate ones
+static int forward(gasp_cnn *c, int n, const float *d_labels, bool stream) {
+    if (stream)
         return c->L == 64   ? forward_stream<6>(c, n, d_labels)
                : c->L == 32 ? forward_stream<5>(c, n, d_labels)
                             : forward_stream<4>(c, n, d_labels);
@@ -936,34 +977,36 @@ static int forward(gasp_cnn *c, int n, const float *d_labels) {
     hipLaunchKernelGGL(conv1_fwd, dim3((unsigned)((tot + 255) / 256)), dim3(256), 0, c->st, c->s, c->w1r, c->p,
                        c->a[1], n, L);
     const int rows = n * L;
+    uint16_t *a4 = c->stream ? c->dz1 : c->a[4];
     for (int k = 2; k <= 4; ++k)
         hipLaunchKernelGGL(conv_mfma<false>, dim3(rows / kConvRows), dim3(256), 0, c->st, c->a[k - 1],
-                           c->wf + (size_t)(k - 2) * 9 * 2 * 64 * 8, c->p + OFF_B[k], (const uint16_t *)nullptr, c->a[k],
-                           n, L);
-    hipLaunchKernelGGL(head, dim3(n), dim3(256), 0, c->st, c->a[4], c->p, d_labels, c->pb, c->loss, c->part_head,
+                           c->wf + (size_t)(k - 2) * 9 * 2 * 64 * 8, c->p + OFF_B[k], (const uint16_t *)nullptr,
+                           k == 4 ? a4 : c->a[k], n, L);
+    hipLaunchKernelGGL(head, dim3(n), dim3(256), 0, c->st, a4, c->p, d_labels, c->pb, c->loss, c->part_head,
                        c->dg, n, L, 1.0f / (float)n);
     CTRY(hipGetLastError());
     return GASP_OK;
 }
 
-// backward after forward(c, n, labels): fills c->g
-static int backward(gasp_cnn *c, int n) {
-    if (c->stream) return backward_stream(c, n, nullptr);
+// backward after forward(c, n, labels, stream): fills c->g
+static int backward(gasp_cnn *c, int n, bool stream) {
+    if (stream) return backward_stream(c, n, nullptr);
     const int L = c->L, N = c->N;
     const size_t tot = (size_t)n * N;
     const int rows = n * L;
     int rc = reduce_to(c, c->part_head, n, HEAD_N, c->g + OFF_FW1);
     if (rc) return rc;
-    hipLaunchKernelGGL(head_bwd_fill, dim3((unsigned)((tot * 16 + 255) / 256)), dim3(256), 0, c->st, c->a[4], c->dg,
-                       c->dz0, n, L);
+    hipLaunchKernelGGL(head_bwd_fill, dim3((unsigned)((tot * 16 + 255) / 256)), dim3(256), 0, c->st,
+                       c->stream ? c->dz1 : c->a[4], c->dg, c->dz0, n, L);
+    float *part = c->stream ? c->parts[2] : c->part;
     uint16_t *dz = c->dz0, *dzn = c->dz1;
     for (int k = 4; k >= 2; --k) {
-        // one partial per workgroup; the buffers hold 4 nmax of them
+        // one partial per workgroup; the buffers hold 4 nmax of them, at most kWgBlocks
         const int nbands = n * (L / 4) * (L / std::min(L, kWgXW));
         const int nblk = std::min({nbands, kWgBlocks, 4 * c->nmax});
-        hipLaunchKernelGGL(conv_wgrad, dim3(nblk), dim3(256), 0, c->st, c->a[k - 1], dz, c->part, n, L);
+        hipLaunchKernelGGL(conv_wgrad, dim3(nblk), dim3(256), 0, c->st, c->a[k - 1], dz, part, n, L);
         // weights and bias are adjacent in the parameter vector
-        if ((rc = reduce_to(c, c->part, nblk, kWgRow, c->g + OFF_W[k])) != 0) return rc;
+        if ((rc = reduce_to(c, part, nblk, kWgRow, c->g + OFF_W[k])) != 0) return rc;
         // d a_{k-1}, masked by a_{k-1} > 0
         hipLaunchKernelGGL(conv_mfma<true>, dim3(rows / kConvRows), dim3(256), 0, c->st, dz,
                            c->wb + (size_t)(k - 2) * 9 * 2 * 64 * 8, (const float *)nullptr, c->a[k - 1], dzn, n, L);
@@ -1009,12 +1052,38 @@ extern "C" int gasp_cnn_predict(gasp_cnn *c, const int8_t *spins, int n, float *
             }
         } else {
             int rc = load_batch(c, spins + (size_t)i0 * c->N, nullptr, nb);
-            if (!rc) rc = forward(c, nb, nullptr);
+            if (!rc) rc = forward(c, nb, nullptr, c->stream);
             if (rc) return rc;
         }
         CTRY(hipMemcpyAsync(pB + i0, c->pb, (size_t)nb * 4, hipMemcpyDeviceToHost, c->st));
     }
     CTRY(hipStreamSynchronize(c->st));
+    uint32_t last = 0u;  // the report stays set: the last grid tells of all
+    if (c->stream && n > 0) memcpy(&last, pB + n - 1, 4);
+    if (last != kNotSpins) return GASP_OK;
+    int rc = to_layers(c);
+    for (int i0 = 0; i0 < n && !rc; i0 += c->nmax) {
+        const int nb = std::min(c->nmax, n - i0);
+        rc = load_batch(c, spins + (size_t)i0 * c->N, nullptr, nb);
+        if (!rc) rc = forward(c, nb, nullptr, false);
+        if (!rc) CTRY(hipMemcpyAsync(pB + i0, c->pb, (size_t)nb * 4, hipMemcpyDeviceToHost, c->st));
+    }
+    if (rc) return rc;
+    CTRY(hipStreamSynchronize(c->st));
+    return GASP_OK;
+}
+
+// The losses of the last forward with labels (waits for it), and whether it was a
+// streamed one of other values than +-1.
+static int get_losses(gasp_cnn *c, int n, double *sum, bool *odd) {
+    std::vector<float> l((size_t)n + 1);
+    CTRY(hipMemcpyAsync(l.data(), c->odd, l.size() * 4, hipMemcpyDeviceToHost, c->st));
+    CTRY(hipStreamSynchronize(c->st));
+    int flag;
+    memcpy(&flag, l.data(), 4);
+    *odd = flag != 0;
+    *sum = 0.0;
+    for (int k = 1; k <= n; ++k) *sum += l[k];
     return GASP_OK;
 }
 
@@ -1024,31 +1093,30 @@ extern "C" int gasp_cnn_gradient(gasp_cnn *c, const int8_t *spins, const float *
     if (!c || !spins || !labels || !grad) return set_error(GASP_ERR_ARG, "gasp_cnn_gradient: bad argument");
     if (!c->weights_ready) return set_error(GASP_ERR_ARG, "gasp_cnn_gradient: parameters not set");
     int rc = load_batch(c, spins, labels, n);
-    if (!rc) rc = forward(c, n, c->y);
-    if (!rc) rc = backward(c, n);
-    if (rc) return rc;
-    CTRY(hipMemcpyAsync(grad, c->g, NPARAM * 4, hipMemcpyDeviceToHost, c->st));
-    std::vector<float> l(n);
-    CTRY(hipMemcpyAsync(l.data(), c->loss, (size_t)n * 4, hipMemcpyDeviceToHost, c->st));
-    CTRY(hipStreamSynchronize(c->st));
-    if (loss) {
-        double s = 0;
-        for (float x : l) s += x;
-        *loss = (float)(s / n);
+    double s = 0.0;
+    bool odd = false;
+    for (bool stream = c->stream; !rc; stream = false) {
+        rc = forward(c, n, c->y, stream);
+        if (!rc) rc = backward(c, n, stream);
+        if (!rc) CTRY(hipMemcpyAsync(grad, c->g, NPARAM * 4, hipMemcpyDeviceToHost, c->st));
+        if (!rc) rc = get_losses(c, n, &s, &odd);
+        if (rc || !stream || !odd) break;
+        rc = to_layers(c);
     }
+    if (rc) return rc;
+    if (loss) *loss = (float)(s / n);
     return GASP_OK;
 }
 
-// backward and the Adam step
-static int backward_adam(gasp_cnn *c, int n, float lr) {
-    c->step++;
+// backward and Adam step number c->step; `odd`: no step if it is set (streamed only)
+static int backward_adam(gasp_cnn *c, int n, float lr, bool stream, const int *odd) {
     const float b1 = 0.9f, b2 = 0.999f;
     const float c1 = 1.0f - powf(b1, (float)c->step), c2 = 1.0f - powf(b2, (float)c->step);
-    if (c->stream) {
-        const AdamArgs ad = {lr, b1, b2, 1e-8f, c1, c2};
+    if (stream) {
+        const AdamArgs ad = {lr, b1, b2, 1e-8f, c1, c2, odd};
         return backward_stream(c, n, &ad);
     }
-    const int rc = backward(c, n);
+    const int rc = backward(c, n, false);
     if (rc) return rc;
     hipLaunchKernelGGL(adam, dim3((NPARAM + 255) / 256), dim3(256), 0, c->st, c->p, c->g, c->m, c->v, NPARAM, lr, b1,
                        b2, 1e-8f, c1, c2);
@@ -1063,14 +1131,17 @@ extern "C" int gasp_cnn_train_step(gasp_cnn *c, const int8_t *spins, const float
     if (!c || !spins || !labels) return set_error(GASP_ERR_ARG, "gasp_cnn_train_step: bad argument");
     if (!c->weights_ready) return set_error(GASP_ERR_ARG, "gasp_cnn_train_step: parameters not set");
     int rc = load_batch(c, spins, labels, n);
-    if (!rc) rc = forward(c, n, c->y);
-    if (!rc) rc = backward_adam(c, n, lr);
+    if (!rc) c->step++;
+    double s = 0.0;
+    bool odd = false;
+    for (bool stream = c->stream; !rc; stream = false) {
+        rc = forward(c, n, c->y, stream);
+        if (!rc) rc = backward_adam(c, n, lr, stream, c->odd);
+        if (!rc) rc = get_losses(c, n, &s, &odd);
+        if (rc || !stream || !odd) break;
+        rc = to_layers(c);
+    }
     if (rc) return rc;
-    std::vector<float> l(n);
-    CTRY(hipMemcpyAsync(l.data(), c->loss, (size_t)n * 4, hipMemcpyDeviceToHost, c->st));
-    CTRY(hipStreamSynchronize(c->st));
-    double s = 0;
-    for (float x : l) s += x;
     *(loss ? loss : &dummy) = (float)(s / n);
     return GASP_OK;
 }
@@ -1092,7 +1163,18 @@ extern "C" int gasp_cnn_set_data(gasp_cnn *c, const int8_t *spins, const float *
     CTRY(hipMalloc((void **)&c->order, (size_t)count * 4));
     CTRY(hipMemcpyAsync(c->data, spins, (size_t)count * c->N, hipMemcpyHostToDevice, c->st));
     CTRY(hipMemcpyAsync(c->data_y, labels, (size_t)count * 4, hipMemcpyHostToDevice, c->st));
+    int odd = 0;
+    if (c->stream) {
+        const size_t words = (size_t)count * c->N / 16;
+        CTRY(hipMemsetAsync(c->odd, 0, 4, c->st));
+        hipLaunchKernelGGL(find_odd, dim3((unsigned)std::min<size_t>((words + 255) / 256, 2048)), dim3(256), 0, c->st,
+                           (const uint4 *)c->data, words, c->odd);
+        CTRY(hipGetLastError());
+        CTRY(hipMemcpyAsync(&odd, c->odd, 4, hipMemcpyDeviceToHost, c->st));
+        CTRY(hipMemsetAsync(c->odd, 0, 4, c->st));
+    }
     CTRY(hipStreamSynchronize(c->st));
+    c->data_odd = odd != 0;
     c->ndata = count;
     return GASP_OK;
 }
@@ -1106,6 +1188,8 @@ extern "C" int gasp_cnn_train_epoch(gasp_cnn *c, const int *order, int count, in
     if (!c->weights_ready) return set_error(GASP_ERR_ARG, "gasp_cnn_train_epoch: parameters not set");
     for (int i = 0; i < count; ++i)
         if (order[i] < 0 || order[i] >= c->ndata) return set_error(GASP_ERR_ARG, "gasp_cnn_train_epoch: index out of range");
+    const bool stream = c->stream && !c->data_odd;
+    if (const int rc = stream || !c->stream ? GASP_OK : layer_buffers(c)) return rc;
     CTRY(hipMemcpyAsync(c->order, order, (size_t)count * 4, hipMemcpyHostToDevice, c->st));
     // the losses stay on the device until the last batch: nothing waits between
     for (int i0 = 0; i0 < count; i0 += batch) {
@@ -1113,8 +1197,9 @@ extern "C" int gasp_cnn_train_epoch(gasp_cnn *c, const int *order, int count, in
         const size_t words = std::max<size_t>((size_t)nb * c->N / 16, (size_t)nb);
         hipLaunchKernelGGL(gather_batch, dim3((unsigned)((words + 255) / 256)), dim3(256), 0, c->st, c->data,
                            c->data_y, c->order + i0, nb, c->N, c->s, c->y);
-        int rc = forward(c, nb, c->y);
-        if (!rc) rc = backward_adam(c, nb, lr);
+        c->step++;
+        int rc = forward(c, nb, c->y, stream);
+        if (!rc) rc = backward_adam(c, nb, lr, stream, nullptr);
         if (rc) return rc;
         CTRY(hipMemcpyAsync(c->data_loss + i0, c->loss, (size_t)nb * 4, hipMemcpyDeviceToDevice, c->st));
     }

@@ -23,7 +23,10 @@
 //
 // conv1 has one input channel of +-1, so a1 at a position is one of 512 rows,
 // found by the nine spins around it: a table of 512 x 32 bfloat16 takes its
-// place, and layer 2's fragments are read from the table.
+// place, and layer 2's fragments are read from the table.  A batch that holds any
+// other value (net_fwd finds out, `odd`) is evaluated by the separate kernels
+// instead: net_head then writes kNotSpins and net_reduce takes no step, and the
+// host runs the batch again.
 #pragma once
 
 namespace cnn {
@@ -110,10 +113,17 @@ struct NetShape {
     }
 };
 
+// Zero if the four bytes are all +1 or -1: bit 0 set, the others alike.
+__device__ __forceinline__ uint32_t not_spins(uint32_t v) {
+    return ((v ^ (v >> 1)) & 0x7E7E7E7Eu) | (~v & 0x01010101u);
+}
+constexpr uint32_t kNotSpins = 0x7FC51D05u;  // net_head's "pB" of a batch that is not +-1: a NaN
+
 // Spins of a group as one 64-bit mask per row (bit = column, 1 = up) to LDS;
 // absent images give zeros.  One thread per 16 columns: `it` < 4 L.
 template <int LG>
-__device__ __forceinline__ void load_bits(const int8_t *__restrict__ s, int n, int img0, uint32_t to, int it) {
+__device__ __forceinline__ void load_bits(const int8_t *__restrict__ s, int n, int img0, uint32_t to, int it,
+                                          int *__restrict__ odd) {
     constexpr int L = 1 << LG;
     const int row = it >> 2, col = (it & 3) * 16, img = img0 + (col >> LG);
     uint32_t bits = 0u;
@@ -121,6 +131,7 @@ __device__ __forceinline__ void load_bits(const int8_t *__restrict__ s, int n, i
         const u32x4 v = *(const u32x4 *)(s + (size_t)img * (L * L) + row * L + (col & (L - 1)));
 #pragma unroll
         for (int q = 0; q < 4; ++q) bits |= ((((~v[q] >> 7) & 0x01010101u) * 0x01020408u) >> 24 & 0xFu) << (4 * q);
+        if (not_spins(v[0]) | not_spins(v[1]) | not_spins(v[2]) | not_spins(v[3])) *odd = 1;
     }
     lds2_set(to + 8u * (uint32_t)row + 2u * (uint32_t)(it & 3), bits);
 }
@@ -230,7 +241,7 @@ __global__ void __launch_bounds__(kFwdThreads) net_fwd(const int8_t *__restrict_
                                                        uint16_t *__restrict__ a2, uint16_t *__restrict__ a3,
                                                        uint16_t *__restrict__ a4, uint32_t *__restrict__ m4,
                                                        float *__restrict__ pool, uint16_t *__restrict__ tab,
-                                                       uint16_t *__restrict__ code, NetShape g) {
+                                                       uint16_t *__restrict__ code, int *__restrict__ odd, NetShape g) {
     constexpr int L = 1 << LG, N = L * L, kSets = 64 >> LG;  // kSets images in a group
     constexpr int kAcc = TRAIN ? kSets : 1;
     const int tid = threadIdx.x, lane = tid & 63, w4 = (tid >> 6) & 3;
@@ -260,7 +271,7 @@ __global__ void __launch_bounds__(kFwdThreads) net_fwd(const int8_t *__restrict_
             if (TRAIN && blockIdx.x == 0) ((uint32_t *)tab)[nine * 16 + c2] = out;
         }
     }
-    if (tid < 4 * L) load_bits<LG>(s, g.n, g.group(g.unit(0)) * kSets, kFwdBits, tid);
+    if (tid < 4 * L) load_bits<LG>(s, g.n, g.group(g.unit(0)) * kSets, kFwdBits, tid, odd);
     __syncthreads();
     // table offsets of a2 block j's six a1 rows, 4j - 3 .. 4j + 2
     auto codes = [&](const Stream &st, int buf) {
@@ -325,7 +336,7 @@ __global__ void __launch_bounds__(kFwdThreads) net_fwd(const int8_t *__restrict_
             if (layer == 1 && step < total) {
                 // the next unit's spins, then the next block's table offsets
                 if (cs.j == 0 && cs.k + 1 < K && (tid & 255) < 4 * L)
-                    load_bits<LG>(s, g.n, g.group(g.unit(cs.k + 1)) * kSets, kFwdBits + (uint32_t)((cs.k + 1) & 1) * 512u, tid & 255);
+                    load_bits<LG>(s, g.n, g.group(g.unit(cs.k + 1)) * kSets, kFwdBits + (uint32_t)((cs.k + 1) & 1) * 512u, tid & 255, odd);
                 cs.next(P);
                 if (step + 1 < total) codes(cs, (step + 1) & 1);
             }
@@ -423,9 +434,11 @@ template <bool TRAIN, int LG>
 __global__ void __launch_bounds__(64) net_head(const float *__restrict__ pool, const float *__restrict__ p,
                                                const float *__restrict__ labels, float *__restrict__ pb,
                                                float *__restrict__ loss, float *__restrict__ part_head,
-                                               float *__restrict__ dg, NetShape g, float inv_batch) {
+                                               float *__restrict__ dg, const int *__restrict__ odd, NetShape g,
+                                               float inv_batch) {
     __shared__ float gs[C], dh[HID];
     const int img = blockIdx.x, t = threadIdx.x;
+    const bool refuse = !TRAIN && *odd != 0;
     constexpr int L = 1 << LG, kSets = 64 >> LG, kAcc = TRAIN ? kSets : 1, kStrips = L / 16;
     const int group = img / kSets, im = img % kSets;
     if (t < C) {
@@ -448,7 +461,7 @@ __global__ void __launch_bounds__(64) net_head(const float *__restrict__ pool, c
     // addition, and then lanes 32 .. 63 round another way
     z = __uint_as_float((uint32_t)__builtin_amdgcn_readfirstlane((int)__float_as_uint(z))) + p[OFF_FB2];
     const float sig = 1.0f / (1.0f + expf(-z));
-    if (t == 0) pb[img] = sig;
+    if (t == 0) pb[img] = refuse ? __uint_as_float(kNotSpins) : sig;
     if (!TRAIN) return;
     const float y = labels[img];
     if (t == 0) loss[img] = fmaxf(z, 0.f) + log1pf(expf(-fabsf(z))) - y * z;
@@ -735,6 +748,7 @@ struct NetParts {
 };
 struct AdamArgs {
     float lr, b1, b2, eps, c1, c2;
+    const int *odd;  // no step if set (NULL: the data are known to be +-1)
 };
 
 template <bool ADAM>
@@ -777,6 +791,7 @@ __global__ void __launch_bounds__(kRedThreads) net_reduce(NetParts q, float *__r
     const int j = dst + col;
     gout[j] = acc;
     if constexpr (ADAM) {
+        if (ad.odd && *ad.odd) return;
         const float gi = acc;
         const float mi = ad.b1 * m[j] + (1.f - ad.b1) * gi;
         const float vi = ad.b2 * v[j] + (1.f - ad.b2) * gi * gi;

@@ -431,7 +431,9 @@ int gasp_autotune(int method, int L, int ngrids, double beta, double h, int prob
  * 3x3 CNN (32 channels) + global average pool + MLP (64) + sigmoid mapping an
  * L x L spin grid (L a power of two >= 16) to pB, trained with binary
  * cross-entropy on shooting labels.  BF16 MFMA kernels with FP32
- * accumulation, FP32 master weights, Adam.  Spins are int8 +-1 [n][L][L];
+ * accumulation, FP32 master weights, Adam.  Spins are int8 +-1 [n][L][L]; a
+ * batch with other values is evaluated on them (for L <= 64 on the slower
+ * kernels of a layer each), conv1's weight gradient on their signs (> 0: +1);
  * parameters a float32 vector of gasp_cnn_num_params() entries. */
 typedef struct gasp_cnn gasp_cnn;
 int gasp_cnn_num_params(void);
