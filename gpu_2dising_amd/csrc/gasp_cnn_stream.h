@@ -13,9 +13,11 @@
 //    gradient, layer 2 makes a1 from the indices;
 //  - net_reduce sums every layer's partial gradients and, in training, applies
 //    Adam and writes the new weights' fragments.
-// Every sum is taken in the order of the separate kernels (a tap after the
-// other, bands of four rows in chains, partials in chunks of 32), so activations,
-// gradients and trained weights are theirs bit for bit.
+// In training every sum is taken in the order of the separate kernels (a tap after
+// the other, bands of four rows in chains, partials in chunks of 32), so activations,
+// gradients and trained weights are theirs bit for bit.  Inference has the same
+// activations, but pools them by eight rows (net_fwd): a grid's pB is the same bits
+// whatever the batch, and differs from the separate kernels' by float32 rounding.
 //
 // The four 16-byte chunks of a position p (64 bytes) lie in LDS at chunk ^ ((p >>
 // 2) & 3), which puts the fragment reads of 16 consecutive positions on 16
@@ -209,6 +211,18 @@ __device__ __forceinline__ void conv_block(const u32x4 (&wa)[9][2], F frag, D do
     }
     done(R - 1, acc[R - 1]);
 }
+// Sum over the 16 lanes of a row, the butterfly over lane ^ 1, 2, 4 and 8 (once the
+// lanes of a quad agree, a mirrored half row gives what lane ^ 4 holds).
+template <int CTRL>
+__device__ __forceinline__ float dpp_move(float v) {
+    return __uint_as_float((uint32_t)__builtin_amdgcn_update_dpp(0, (int)__float_as_uint(v), CTRL, 0xf, 0xf, true));
+}
+__device__ __forceinline__ float sum16(float v) {
+    v += dpp_move<0xB1>(v);    // quad_perm [1, 0, 3, 2]
+    v += dpp_move<0x4E>(v);    // quad_perm [2, 3, 0, 1]
+    v += dpp_move<0x141>(v);   // row_half_mirror
+    return v + dpp_move<0x140>(v);  // row_mirror
+}
 // OR of a value over the four lanes of a position (lane, lane ^ 16, ^ 32, ^ 48)
 __device__ __forceinline__ uint32_t or_quarters(uint32_t m) {
     const auto x = __builtin_amdgcn_permlane16_swap(m, m, false, false);
@@ -230,8 +244,12 @@ __device__ __forceinline__ uint32_t or_quarters(uint32_t m) {
 // against 372 + 3 x 663 + 198 for the layers one by one.  The first form took 834:
 // conv2's waves made the table offsets themselves, rows of the table that grids
 // need together shared banks, and a step's reads went out as they were needed.
-// pool[unit][wave][set][32]: sums of a4 over a wave's 16 columns and the unit's
-// rows, in training those of each residue mod 64 / L apart (as `head` adds them).
+// pool, training: [unit][wave][set][32], sums of a4 over a wave's 16 columns and
+// the unit's rows, those of each residue mod 64 / L apart (as `head` adds them).
+// pool, inference: [group][eight rows][wave][32], so that an image's sums do not
+// depend on the bands that the number of images leads to (with a sum per unit,
+// summed through LDS, 4096 grids took as long: 938 us a call against 925, and a
+// grid's pB moved in its last bits with the size of the batch).
 // a4: only where bands leave the pooling to `head` (else NULL).
 // m4[image][position]: bit c set where a4 > 0.  tab, code: conv1's table and every
 // position's index in it, for net_back<2>.
@@ -405,14 +423,14 @@ __global__ void __launch_bounds__(kFwdThreads) net_fwd(const int8_t *__restrict_
                             if (a4 && img < g.n) *(u32x4 *)(a4 + pos * C + 8 * oc) = to_chunk(x[0], y[0], x[1], y[1]);
                         }
                     });
-                    if (st.j == P - 2) {  // the unit's last block
+                    // training: the unit's last block; inference: every eight rows
+                    if (TRAIN ? st.j == P - 2 : (st.j & 1) != 0) {
+                        const size_t to = TRAIN ? (size_t)u : (size_t)g.group(u) * (L / 8) + (size_t)(y0 + 4 * st.j) / 8;
 #pragma unroll
                         for (int q = 0; q < 8 * kAcc; ++q) {
-                            float v = psum[q / 8][q % 8];
-#pragma unroll
-                            for (int o = 1; o < 16; o <<= 1) v += __shfl_xor(v, o, 64);
+                            const float v = sum16(psum[q / 8][q % 8]);
                             const int e = q % 8;
-                            if (pl == 0) pool[(((size_t)u * 4 + w4) * kAcc + q / 8) * C + 16 * (e >> 2) + 4 * kq + (e & 3)] = v;
+                            if (pl == 0) pool[((to * 4 + w4) * kAcc + q / 8) * C + 16 * (e >> 2) + 4 * kq + (e & 3)] = v;
                             psum[q / 8][q % 8] = 0.f;
                         }
                     }
@@ -443,10 +461,11 @@ __global__ void __launch_bounds__(64) net_head(const float *__restrict__ pool, c
     const int group = img / kSets, im = img % kSets;
     if (t < C) {
         float v = 0.f;
-        for (int b = 0; b < g.nb; ++b)
+        const int parts = TRAIN ? g.nb : L / 8;
+        for (int b = 0; b < parts; ++b)
             for (int q = 0; q < kAcc; ++q)
                 for (int w = 0; w < kStrips; ++w)
-                    v += pool[(((size_t)(group * g.nb + b) * 4 + im * kStrips + w) * kAcc + q) * C + t];
+                    v += pool[(((size_t)group * parts + b) * 4 + im * kStrips + w) * kAcc * C + q * C + t];
         gs[t] = v / (float)(L * L);
     }
     __syncthreads();
