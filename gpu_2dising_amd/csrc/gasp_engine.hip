@@ -1498,6 +1498,8 @@ static int sweep_grids_run(int L, int R, int method, gasp_rng_state *d_state, do
         hipLaunchKernelGGL(pack_bits, bits_grid(R, 32 * sh.stride), blk, 0, st, d_grids, (unsigned *)lat, R, N, sh.stride, 1);
     else if (lay == 0)
         hipLaunchKernelGGL(pack_hbm, grid, blk, 0, st, d_grids, (unsigned char *)lat, R, N, sh.stride, 1);
+    else if (nsweeps == 0)
+        hipLaunchKernelGGL(only_spins, blocks_for((size_t)R * N, 4096), blk, 0, st, d_grids, (size_t)R * N);
     HIP_TRY(hipGetLastError());
     SweepFn fn = sh.win ? window_fn(0, sh.win, sh.wmode, is_pow2(L), WIN_INT32)
                         : sweep_fn(method, 0, sh.S, sh.W, is_pow2(L), sh.stage);
