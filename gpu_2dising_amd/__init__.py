@@ -32,7 +32,7 @@ EXPORTS = (
     "gasp_set_tuning", "gasp_get_tuning", "gasp_get_run_stats", "gasp_set_conflict_filter",
     "gasp_engine_get_conflict_filter", "gasp_set_lattice_staging", "gasp_engine_get_lattice_staging",
     "gasp_set_dependence_tables",
-    "gasp_engine_set_attempt",
+    "gasp_engine_set_attempt", "gasp_get_window", "gasp_engine_get_window",
     "gasp_engine_create", "gasp_engine_destroy", "gasp_engine_set_grids", "gasp_engine_get_grids",
     "gasp_engine_gather_grids", "gasp_engine_get_gridstates",
     "gasp_engine_set_inputs", "gasp_engine_set_freeze",
@@ -135,6 +135,8 @@ def lib() -> C.CDLL:
     L.gasp_set_lattice_staging.argtypes = [C.c_int]
     L.gasp_set_dependence_tables.argtypes = [C.c_int]
     L.gasp_get_tuning.argtypes = [C.c_int, C.c_int, C.c_int, ip, ip]
+    L.gasp_get_window.argtypes = [C.c_int, C.c_int, C.c_int, ip, ip]
+    L.gasp_get_window.restype = None
     L.gasp_get_run_stats.argtypes = [C.POINTER(RunStats)]
     L.gasp_engine_create.argtypes = [C.c_int, C.c_int, C.c_int, vp, C.c_double, C.c_double,
                                      C.POINTER(vp)]
@@ -163,6 +165,8 @@ def lib() -> C.CDLL:
     L.gasp_engine_kernel_ms.argtypes = [vp]
     L.gasp_engine_kernel_ms.restype = C.c_double
     L.gasp_engine_get_shape.argtypes = [vp, C.POINTER(C.c_int), C.POINTER(C.c_int)]
+    L.gasp_engine_get_window.argtypes = [vp, ip, ip]
+    L.gasp_engine_get_window.restype = C.c_int
     L.gasp_engine_get_conflict_filter.argtypes = [vp, C.POINTER(C.c_int)]
     L.gasp_engine_get_lattice_staging.argtypes = [vp, C.POINTER(C.c_int)]
     L.gasp_engine_set_attempt.argtypes = [vp, C.c_ulonglong]
@@ -330,6 +334,12 @@ class Engine:
         s, w = C.c_int(0), C.c_int(0)
         check(lib().gasp_engine_get_shape(self.ptr, C.byref(s), C.byref(w)))
         return s.value, w.value
+
+    def window(self) -> tuple:
+        """(waves per replica, key-table entries) of the kernel of one replica per workgroup; (0, 0): another kernel."""
+        w, t = C.c_int(0), C.c_int(0)
+        check(lib().gasp_engine_get_window(self.ptr, C.byref(w), C.byref(t)))
+        return w.value, t.value
 
     def lattice_staging(self) -> int:
         """The engine's lattice staging: 1 in HBM, 2 staged in LDS as bytes, 3 as bits (method 0 over several waves)."""
@@ -509,6 +519,13 @@ def get_tuning(method: int, L: int, ngrids: int) -> tuple[int, int]:
     s, w = C.c_int(), C.c_int()
     lib().gasp_get_tuning(method, L, ngrids, C.byref(s), C.byref(w))
     return s.value, w.value
+
+
+def get_window(method: int, L: int, ngrids: int) -> tuple[int, int]:
+    """As Engine.window, for engines of (method, L, ngrids) at the present settings."""
+    w, t = C.c_int(), C.c_int()
+    lib().gasp_get_window(method, L, ngrids, C.byref(w), C.byref(t))
+    return w.value, t.value
 
 
 def run_stats() -> RunStats:

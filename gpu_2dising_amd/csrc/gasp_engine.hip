@@ -735,6 +735,16 @@ static int launch_shape(int method, int L, int R, LaunchShape *sh) {
     return GASP_OK;
 }
 
+extern "C" void gasp_get_window(int method, int L, int ngrids, int *waves, int *table_entries) {
+    LaunchShape sh;
+    if (method < 0 || method > 3 || L < 2 || L > 8192 || ngrids < 1 || launch_shape(method, L, ngrids, &sh)) {
+        clear_error();
+        sh = LaunchShape{};
+    }
+    if (waves) *waves = sh.win;
+    if (table_entries) *table_entries = sh.win && sh.wmode == WIN_TABLE ? sh.tbl : 0;
+}
+
 // LDS of a split-word workgroup (W = 2, 4, 8: 4, 2, 1 bytes per site) with the mark plane
 static size_t marks_lds_bytes(int moff, int W, int stride) {
     return (size_t)kLdsLattice + (size_t)moff + (size_t)(8 / W) * (size_t)stride;
@@ -1445,6 +1455,13 @@ extern "C" int gasp_engine_get_shape(gasp_engine *e, int *slots, int *waves) {
     if (!e || !slots || !waves) return set_error(GASP_ERR_ARG, "gasp_engine_get_shape: NULL argument");
     *slots = e->S;
     *waves = e->W;
+    return GASP_OK;
+}
+
+extern "C" int gasp_engine_get_window(gasp_engine *e, int *waves, int *table_entries) {
+    if (!e || !waves || !table_entries) return set_error(GASP_ERR_ARG, "gasp_engine_get_window: NULL argument");
+    *waves = e->win;
+    *table_entries = e->win && e->wmode == WIN_TABLE ? e->tbl : 0;
     return GASP_OK;
 }
 

@@ -232,6 +232,9 @@ void gasp_free(void *d_ptr);
 void gasp_set_tuning(int slots_per_replica, int waves_per_group);
 void gasp_get_tuning(int method, int L, int ngrids, int *slots_per_replica,
                      int *waves_per_group);
+/* As gasp_engine_get_window, for an engine or gasp_sweep_grids call of
+ * (method, L, ngrids) at the present settings. */
+void gasp_get_window(int method, int L, int ngrids, int *waves, int *table_entries);
 
 /* Conflict filter of method 2 on split words (half words with 2 to 32 slots;
  * quarter and eighth words with 8 to 32 slots and Philox streams), for
@@ -372,6 +375,11 @@ void *gasp_engine_stream(gasp_engine *e);
 /* The engine's launch shape: slots per replica and waves per workgroup (the
  * word split for method 2), as gasp_set_tuning takes them. */
 int gasp_engine_get_shape(gasp_engine *e, int *slots, int *waves);
+/* Whether the engine runs the kernel of one replica per workgroup (see
+ * gasp_set_tuning): the waves per replica (1, 2, 4 or 8; 0: another kernel)
+ * and the entries of its key table in LDS (0: a dword per site holds spin and
+ * key). */
+int gasp_engine_get_window(gasp_engine *e, int *waves, int *table_entries);
 /* Moves the engine's replicas to per-replica attempt `attempt` of their
  * Philox streams (the next sweep uses attempts attempt, attempt + 1, ...):
  * rewinding replays a trajectory's random numbers.  Waits for the engine's
