@@ -58,3 +58,39 @@ def test_other_values_count_as_down(gpu, engine_lib, oracle, automatic, explicit
         rng.free()
         G.lib().gasp_free(d)
         G.lib().gasp_free(d_mag)
+
+
+# explicit shapes; 256 slots spread a method-0 replica over four waves; and counts above the lines of the one-replica kernel
+@pytest.mark.parametrize("method,L,R,shape", [(0, 64, 9, (256, 4)), (0, 17, 50, (16, 1)), (1, 24, 70, (16, 2)),
+                                              (1, 33, 100, (8, 1)), (2, 64, 130, (16, 2)), (2, 33, 70, (8, 1)),
+                                              (2, 32, 200, (16, 4)), (2, 48, 1000, (16, 2)), (0, 9, 16500, None),
+                                              (1, 9, 16500, None), (2, 9, 16500, None)])
+@pytest.mark.parametrize("noalloc", [False, True])
+def test_native_layout_route(gpu, engine_lib, oracle, automatic, noalloc, method, L, R, shape):
+    """Two calls in a row with a magnetisation buffer, then one without, which moves the lattice in the workspace."""
+    G, O = engine_lib, oracle
+    if shape:
+        G.set_tuning(*shape)
+    assert G.get_window(method, L, R) == (0, 0)
+    print(f"[routes native] method={method} L={L} R={R} shape={shape} noalloc={noalloc}", flush=True)
+    fn = G.lib().gasp_sweep_grids_noalloc if noalloc else G.lib().gasp_sweep_grids
+    rs = np.random.default_rng(L + R)
+    want = np.where(rs.random((R, L, L)) < 0.35, 1, -1).astype(np.int32)
+    got, mag = np.empty_like(want), np.empty(R, np.float32)
+    d, d_mag = _device_grids(G, want), _device_grids(G, np.zeros((R, 1, 1), np.int32))
+    rng = G.RngState(R, 77)
+    at = 0
+    try:
+        for n, with_mag in ((2, True), (1, True), (1, False)):
+            G.check(fn(L, R, method, rng.ptr, BETA, H, d, n, d_mag if with_mag else None, None))
+            want = O.sweep_philox(L, want, 77, at, n * L * L, BETA, H)
+            at += n * L * L
+            G._d2h(got, d)
+            assert np.array_equal(got, want), (n, with_mag)
+            if with_mag:
+                G._d2h(mag, d_mag)
+                assert np.array_equal(mag, _mag(want)), n
+    finally:
+        rng.free()
+        G.lib().gasp_free(d)
+        G.lib().gasp_free(d_mag)
