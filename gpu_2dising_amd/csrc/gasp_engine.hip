@@ -320,7 +320,7 @@ static size_t sliced_lds_bytes(int N) { return (size_t)kSlLat + (size_t)kSlEntry
 // explicit gasp_set_tuning override is active.
 struct TunedShape {
     int S, W;
-    bool window;  // the automatic sweep_window was faster than (S, W)
+    int window;  // the automatic sweep_window was timed against (S, W): 1 faster, -1 slower; 0: not timed
 };
 static std::map<std::tuple<int, int, int>, TunedShape> g_tuned;
 
@@ -645,7 +645,7 @@ static void window_shape(int method, int L, int R, LaunchShape *sh) {
         (g_tune_stage >= 1 && g_tune_stage <= 3) || g_tune_tables > 0)
         return;
     auto it = g_tuned.find(std::make_tuple(method, L, R));
-    if (it != g_tuned.end() && !it->second.window) return;
+    if (it != g_tuned.end() && it->second.window < 0) return;
     const long long ncu = sh->ncu;
     const long long per_cu = L > 64 ? 40 : method == 2 && L > 32 ? 52 : 64;
     if (!(method == 0 && L >= 32) && R > per_cu * ncu) return;
@@ -1964,15 +1964,21 @@ extern "C" int gasp_autotune(int method, int L, int ngrids, double beta, double 
         }
     }
     // sweep_window, which no (S, W) names, where the automatic choice takes it
-    bool window = false;
-    g_tuned.erase(std::make_tuple(method, L, ngrids));
+    // (an explicit filter, staging or table setting bars it here: then what an
+    // earlier call found stands)
+    const auto key = std::make_tuple(method, L, ngrids);
+    const auto known = g_tuned.find(key);
+    int window = known == g_tuned.end() ? 0 : known->second.window;
+    bool faster = false;  // here and now
+    g_tuned.erase(key);
     g_tune_slots = g_tune_waves = 0;
     {
         gasp_engine *e = nullptr;
         if (!engine_new(L, ngrids, method, rng, thr, 0, beta, h, &e)) {
             if (e->win) {
                 const double rate = probe_rate(e, grids, ngrids, probe_sweeps, probe_sweeps);
-                window = rate > best;
+                faster = rate > best;
+                window = faster ? 1 : -1;
                 best = std::max(rate, best);
             }
             engine_free(e);
@@ -1982,7 +1988,7 @@ extern "C" int gasp_autotune(int method, int L, int ngrids, double beta, double 
     }
     int blaunch = check_sweeps;
     if (best > 0 && check_sweeps > 1) {
-        if (!window) {
+        if (!faster) {
             g_tune_slots = bs;
             g_tune_waves = bw;
         }
@@ -2006,7 +2012,7 @@ extern "C" int gasp_autotune(int method, int L, int ngrids, double beta, double 
     g_tune_waves = save_w;
     (void)hipFree(rng);
     if (best < 0) return set_error(GASP_ERR_ARG, "gasp_autotune: no candidate ran");
-    g_tuned[std::make_tuple(method, L, ngrids)] = {bs, bw, window};
+    g_tuned[key] = {bs, bw, window};
     if (best_slots) *best_slots = bs;
     if (best_waves) *best_waves = bw;
     if (best_launch_sweeps) *best_launch_sweeps = blaunch;
