@@ -12,7 +12,7 @@ from dataclasses import dataclass, field
 
 import numpy as np
 
-from . import (CHECK_COUNT, CHECK_FATES, Engine, Graph, RngState, autotune, set_conflict_filter,
+from . import (CHECK_COUNT, CHECK_FATES, Engine, Graph, RngState, autotune, get_window, set_conflict_filter,
                set_dependence_tables, set_lattice_staging, set_tuning)
 
 # L, replicas, gpu_method: four lattice sizes on the LDS multispin path and
@@ -40,7 +40,7 @@ class Group:
     h: float
     itask: int
     seed: int
-    slots: int = 0
+    slots: int = 0  # 0, 0: automatic (of the tuner: the kernel of one replica per workgroup)
     waves: int = 0
     launch_sweeps: int = 0
     probe_rate: float = 0.0
@@ -82,6 +82,9 @@ class Batch:
         4.59-4.61 ms with the plane on every method-2 group, 4.70 on L = 32
         and 96, 4.90 on L = 32 only; on bits beside 16384 entries (the
         engine's own choice, 140 KB) 5.57 ms.
+        With all three at 0, groups of few replicas run the kernel of one
+        replica per workgroup where the tuner finds it faster; their slots and
+        waves are then 0, and `refine` leaves them there.
         `refine`: after the per-group tuning, a coordinate search over the
         groups' shapes on the captured graph itself (see `_refine`)."""
         filters = ([2 if m == 2 else 1 for (_, _, m) in groups] if conflict_filter is None else
@@ -115,6 +118,9 @@ class Batch:
                 g.slots, g.waves, g.launch_sweeps = shapes[k]
             elif tune:
                 g.slots, g.waves, g.launch_sweeps, g.probe_rate = autotune(m, L, R, probe_sweeps, beta, h, chk)
+                if get_window(m, L, R)[0]:
+                    # the tuner found the one-replica kernel faster than the shape it returns
+                    g.slots, g.waves, g.launch_sweeps = 0, 0, chk
             else:
                 g.launch_sweeps = chk
             self.groups.append(g)
@@ -187,6 +193,8 @@ class Batch:
         return (self.graph.ms() - ms0) / replays
 
     def _candidates(self, g: Group) -> list:
+        if g.slots == 0:  # automatic: no shape names its kernel
+            return []
         if g.method == 0 and g.slots > 64:
             return [(s_, s_ // 64, k) for s_ in (256, 512) for k in (self.chk // 4, self.chk // 2, self.chk)
                     if k >= 1 and self.chk % k == 0]
@@ -226,7 +234,9 @@ class Batch:
         ends = [(best, [shape(g) for g in self.groups])]
         second = []
         for g, sh in zip(self.groups, tuned):
-            if g.method == 2:
+            if g.slots == 0:
+                second.append(sh)
+            elif g.method == 2:
                 second.append((sh[0], sh[1], self.chk))
             elif g.method == 0 and g.slots > 64:
                 second.append(max(self._candidates(g), key=lambda c: (c[0], -c[2])))

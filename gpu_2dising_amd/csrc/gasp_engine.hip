@@ -1963,24 +1963,19 @@ extern "C" int gasp_autotune(int method, int L, int ngrids, double beta, double 
             bw = W;
         }
     }
-    // sweep_window, which no (S, W) names, where the automatic choice takes it
-    // (an explicit filter, staging or table setting bars it here: then what an
-    // earlier call found stands)
+    // sweep_window, which no (S, W) names, where the automatic choice takes it: later
+    // automatic engines run it if it was faster.  What is returned belongs to (bs,
+    // bw), the shape that gasp_set_tuning can ask for.  (An explicit filter, staging or table setting bars it here: then what an
+    // earlier call found stands.)
     const auto key = std::make_tuple(method, L, ngrids);
     const auto known = g_tuned.find(key);
     int window = known == g_tuned.end() ? 0 : known->second.window;
-    bool faster = false;  // here and now
     g_tuned.erase(key);
     g_tune_slots = g_tune_waves = 0;
     {
         gasp_engine *e = nullptr;
         if (!engine_new(L, ngrids, method, rng, thr, 0, beta, h, &e)) {
-            if (e->win) {
-                const double rate = probe_rate(e, grids, ngrids, probe_sweeps, probe_sweeps);
-                faster = rate > best;
-                window = faster ? 1 : -1;
-                best = std::max(rate, best);
-            }
+            if (e->win) window = probe_rate(e, grids, ngrids, probe_sweeps, probe_sweeps) > best ? 1 : -1;
             engine_free(e);
         } else {
             clear_error();
@@ -1988,10 +1983,8 @@ extern "C" int gasp_autotune(int method, int L, int ngrids, double beta, double 
     }
     int blaunch = check_sweeps;
     if (best > 0 && check_sweeps > 1) {
-        if (!faster) {
-            g_tune_slots = bs;
-            g_tune_waves = bw;
-        }
+        g_tune_slots = bs;
+        g_tune_waves = bw;
         gasp_engine *e = nullptr;
         if (!engine_new(L, ngrids, method, rng, thr, 0, beta, h, &e)) {
             double best_l = -1.0;

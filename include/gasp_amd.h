@@ -430,7 +430,12 @@ int gasp_bootstrap_errbar_libc(const int *fates, int ninputs, int n, int m, unsi
  * of that (method, L, ngrids).  With check_sweeps > 0 it then times that
  * interval as 1, 2, 4, ... equal launches (of at least check_sweeps / 8
  * sweeps) and returns the fastest sweeps per launch in *best_launch_sweeps
- * (check_sweeps when 0 or 1).  *best_rate: attempts/s of the chosen shape. */
+ * (check_sweeps when 0 or 1).  *best_rate: attempts/s of the chosen shape.
+ * The kernel of one replica per workgroup, which no shape names, is timed too
+ * where the automatic choice takes it: if it was faster, later engines at
+ * automatic settings run it (gasp_get_window tells), and the results returned
+ * are still the fastest shape's.  To have that kernel, leave gasp_set_tuning
+ * at (0, 0); the returned shape asks for the slower one. */
 int gasp_autotune(int method, int L, int ngrids, double beta, double h, int probe_sweeps, int check_sweeps,
                   int *best_slots, int *best_waves, int *best_launch_sweeps, double *best_rate);
 
