@@ -1073,9 +1073,13 @@ static int engine_advance(gasp_engine *e, uint64_t n, int check, double dn, doub
         const uint64_t nb = std::min(left, cap);
         if (e->rng.kind == KIND_MT) {
             uint32_t *st = (uint32_t *)((char *)e->d_rng + kRngMtOffset);
-            hipLaunchKernelGGL(mt_draws_kernel, dim3(e->R), dim3(256), 0, e->stream, st, e->R,
-                               3ull * e->rng.attempts, 3ull * nb, e->d_draws);
-            HIP_TRY(hipGetLastError());
+            // a launch has fewer than 2^32 work-items; the kernel's replica r is word r of each row of `st`
+            const unsigned most = 0xffffffffu / 256, R = (unsigned)e->R;
+            for (unsigned r0 = 0; r0 < R; r0 += most) {
+                hipLaunchKernelGGL(mt_draws_kernel, dim3(std::min(R - r0, most)), dim3(256), 0, e->stream, st + r0, e->R,
+                                   3ull * e->rng.attempts, 3ull * nb, e->d_draws + (size_t)r0 * (3ull * nb));
+                HIP_TRY(hipGetLastError());
+            }
         }
         const int rc = launch_sweep(e, nb, e->rng.kind == KIND_MT ? e->d_draws : nullptr,
                                     left == nb ? check : CHECK_NONE, dn, up);
