@@ -675,6 +675,7 @@ static void window_shape(int method, int L, int R, LaunchShape *sh) {
         const int waves = res * w;
         if ((128 * w <= E / 8 && waves <= (w == 2 ? 34 : 28)) || (128 * w <= E / 4 && waves <= 8)) W = w;
     }
+    if ((uint64_t)R * 64u * (uint64_t)W > 0xffffffffull) return;  // more work-items than one launch may have
     sh->win = W;
     sh->wmode = M > 0 ? WIN_TABLE : WIN_PACKED;
     sh->tbl = std::max(M, 1);

@@ -29,6 +29,12 @@ def test_method_0_and_3(engine_lib):
     assert engine_lib.get_window(0, 1, 64) == (0, 0) and engine_lib.get_window(5, 32, 64) == (0, 0)
 
 
+def test_one_launch(engine_lib):
+    """One wave per replica at L = 32: a launch has fewer than 2^32 work-items."""
+    assert engine_lib.get_window(0, 32, 2**26 - 1)[0] == 1
+    assert engine_lib.get_window(0, 32, 2**26) == (0, 0)
+
+
 @pytest.mark.parametrize("method", [0, 1, 2])
 @pytest.mark.parametrize("setting,value", [("set_tuning", (16, 2)), ("set_tuning", (16, 0)), ("set_tuning", (0, 2)),
                                            ("set_conflict_filter", (1,)), ("set_conflict_filter", (2,)),
