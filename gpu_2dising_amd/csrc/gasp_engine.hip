@@ -2275,8 +2275,8 @@ extern "C" void mc_driver_gpu(mc_gpu_grids_t grids, double beta, double h, int *
     t_stats.sweep_kernel_ms = e->kernel_ms - t_ms0;
     t_stats.attempts_per_replica = (double)(e->rng.attempts);
     t_stats.launches = e->launches;
-    t_stats.slots_per_replica = e->S;
-    t_stats.waves_per_group = e->W;
+    t_stats.slots_per_replica = e->win ? 64 * e->win : e->S;
+    t_stats.waves_per_group = e->win ? e->win : e->W;
     t_stats.method = e->method;
     engine_free(e);
     if (!rc && dumped) {

@@ -270,7 +270,9 @@ void gasp_set_dependence_tables(int max_entries);
 
 /* Statistics of the most recent mc_driver_gpu / gasp_engine run on this
  * thread: sweep-kernel time (HIP events), attempts performed per replica,
- * kernel launches. */
+ * kernel launches, and the shape of the kernel that ran (as gasp_set_tuning
+ * takes it; for the kernel of one replica per workgroup, which it cannot name,
+ * the lanes and waves of a replica). */
 typedef struct {
     double sweep_kernel_ms;
     double attempts_per_replica;

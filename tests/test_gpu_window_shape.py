@@ -47,3 +47,24 @@ def test_both_sides_of_the_table(gpu, engine_lib, oracle, L, mt):
     rng.free()
     ref = O.sweep_mt_per_replica(L, g0.copy(), 3, 3, 0.3, 0.07) if mt else O.sweep_philox(L, g0.copy(), 3, 0, 3 * L * L, 0.3, 0.07)
     assert np.array_equal(got, ref)
+
+
+@pytest.mark.parametrize("method,L,R", [(2, 32, 100), (1, 64, 9), (0, 45, 20)])
+@pytest.mark.parametrize("shape", [(0, 0), (16, 2)])
+def test_run_statistics(gpu, engine_lib, shape, method, L, R):
+    """A driver run reports the shape of the kernel that ran."""
+    G = engine_lib
+    print(f"[window stats] method={method} L={L} R={R} shape={shape}", flush=True)
+    rng = G.RngState(R, 1)
+    G.set_tuning(*shape)
+    try:
+        waves = G.get_window(method, L, R)[0]
+        want = (64 * waves, waves) if waves else G.get_tuning(method, L, R)
+        assert (waves > 0) == (shape == (0, 0))
+        st = G.run_driver(L, -np.ones((R, L, L), np.int32), beta=0.3, h=0.07, rng=rng, method=method, tot_nsweeps=4,
+                          mag_output_int=2, grid_output_int=4, itask=0, dn_thr=-0.9, up_thr=0.9, ninputs=1,
+                          outfunc=lambda *a: 0)["stats"]
+    finally:
+        G.set_tuning(0, 0)
+        rng.free()
+    assert (st.slots_per_replica, st.waves_per_group) == want and st.method == method
