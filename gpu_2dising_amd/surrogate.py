@@ -201,7 +201,8 @@ def estimate(grids, params, *, lo=0.2, hi=0.8, reps=128, seed=303, max_sweeps=20
     the shooting standard error by sqrt(0.25 / 128) = 0.044."""
     L = grids.shape[1]
     t0 = time.perf_counter()
-    net = Surrogate(L, 4096)
+    # one for 4096 grids a batch holds 4.4 GB at L = 64 and takes milliseconds to make and close
+    net = Surrogate(L, min(4096, max(1, len(grids))))
     net.set_params(params)
     pred = net.predict(grids)
     net.close()
