@@ -247,9 +247,10 @@ __device__ __forceinline__ uint32_t or_quarters(uint32_t m) {
 // pool, training: [unit][wave][set][32], sums of a4 over a wave's 16 columns and
 // the unit's rows, those of each residue mod 64 / L apart (as `head` adds them).
 // pool, inference: [group][eight rows][wave][32], so that an image's sums do not
-// depend on the bands that the number of images leads to (with a sum per unit,
-// summed through LDS, 4096 grids took as long: 938 us a call against 925, and a
-// grid's pB moved in its last bits with the size of the batch).
+// depend on the bands that the number of images leads to (with a sum per unit a
+// grid's pB moved in its last bits with the size of the batch).  Written 16 bytes a
+// lane that costs nothing: 1024 grids of L = 64 180 us, 181 with a sum per unit,
+// 185 written 4 bytes a lane.
 // a4: only where bands leave the pooling to `head` (else NULL).
 // m4[image][position]: bit c set where a4 > 0.  tab, code: conv1's table and every
 // position's index in it, for net_back<2>.
@@ -426,12 +427,16 @@ __global__ void __launch_bounds__(kFwdThreads) net_fwd(const int8_t *__restrict_
                     // training: the unit's last block; inference: every eight rows
                     if (TRAIN ? st.j == P - 2 : (st.j & 1) != 0) {
                         const size_t to = TRAIN ? (size_t)u : (size_t)g.group(u) * (L / 8) + (size_t)(y0 + 4 * st.j) / 8;
+                        f32x4 *out = (f32x4 *)(pool + (to * 4 + w4) * kAcc * C + 4 * kq);
 #pragma unroll
-                        for (int q = 0; q < 8 * kAcc; ++q) {
-                            const float v = sum16(psum[q / 8][q % 8]);
-                            const int e = q % 8;
-                            if (pl == 0) pool[((to * 4 + w4) * kAcc + q / 8) * C + 16 * (e >> 2) + 4 * kq + (e & 3)] = v;
-                            psum[q / 8][q % 8] = 0.f;
+                        for (int q = 0; q < 2 * kAcc; ++q) {
+                            f32x4 v;
+#pragma unroll
+                            for (int j = 0; j < 4; ++j) {
+                                v[j] = sum16(psum[q / 2][4 * (q & 1) + j]);
+                                psum[q / 2][4 * (q & 1) + j] = 0.f;
+                            }
+                            if (pl == 0) out[4 * q] = v;
                         }
                     }
                 }
