@@ -1153,6 +1153,7 @@ extern "C" int gasp_cnn_train_step(gasp_cnn *c, const int8_t *spins, const float
 extern "C" int gasp_cnn_set_data(gasp_cnn *c, const int8_t *spins, const float *labels, int count) {
     gasp::clear_error();
     if (!c || !spins || !labels || count < 1) return set_error(GASP_ERR_ARG, "gasp_cnn_set_data: bad argument");
+    c->ndata = 0;  // none until the new ones are there
     cfree(c->data);
     cfree(c->data_y);
     cfree(c->data_loss);

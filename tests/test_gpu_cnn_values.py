@@ -81,3 +81,23 @@ def test_training(gpu, engine_lib):
     assert np.max(np.abs(one - ref)) < 1e-6
     assert np.array_equal(a, b)
     assert abs(mean - (32 * losses[0] + 32 * losses[1] + 6 * losses[2]) / 70) < 1e-6
+
+
+def test_data_that_do_not_fit(gpu, engine_lib):
+    """Training data beyond the device's memory are refused, and epochs with them, until there are some again."""
+    import ctypes as C
+
+    G = engine_lib
+    K, p, spins, y = _case(64, 6, 14)
+    print("[values data]", flush=True)
+    order = np.arange(6, dtype=np.int32)
+    with G.Surrogate(64, 6) as net:
+        net.set_params(p)
+        net.set_data(spins, y)
+        rc = G.lib().gasp_cnn_set_data(net.ptr, spins.ctypes.data_as(C.POINTER(C.c_int8)),
+                                       y.ctypes.data_as(C.POINTER(C.c_float)), 2**31 - 1)  # 8.8 TB, refused before it is read
+        assert rc != 0
+        with pytest.raises(G.GaspError):
+            net.train_epoch(order, 6, 1e-3)
+        with pytest.raises(G.GaspError):
+            net.train_epoch(order[:1], 1, 1e-3)
