@@ -42,6 +42,9 @@ int set_error(int code, const char *fmt, ...) {
     t_msg = buf;
     fprintf(stderr, "%s\n", buf);
     fflush(stderr);
+    // HIP keeps the error of a failed call until it is asked for: it would be taken
+    // for that of the next call's launches
+    if (code == GASP_ERR_HIP || code == GASP_ERR_NOMEM) (void)hipGetLastError();
     return code;
 }
 void clear_error() {
