@@ -23,6 +23,9 @@
 // 2) & 3), which puts the fragment reads of 16 consecutive positions on 16
 // different bank quads.
 //
+// L <= 64, as a ring row holds 64 columns: with 128 the two rings take 200 KB, more
+// than a CU's LDS (strips of columns with halos, which would fit, were not tried).
+//
 // conv1 has one input channel of +-1, so a1 at a position is one of 512 rows,
 // found by the nine spins around it: a table of 512 x 32 bfloat16 takes its
 // place, and layer 2's fragments are read from the table.  A batch that holds any

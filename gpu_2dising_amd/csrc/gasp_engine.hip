@@ -1093,8 +1093,6 @@ static int engine_advance(gasp_engine *e, uint64_t n, int check, double dn, doub
     return GASP_OK;
 }
 
-// Packs int32 grids into the native layout.  `ninputs` grids are given;
-// replica r takes grid r / (R / ninputs) (ninputs == R: one grid per replica).
 static size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 
 // The engine's scratch memory, at least `bytes`: staging of grids, packed records
@@ -1112,6 +1110,8 @@ static int scratch_error(hipError_t he) {
                      hipGetErrorString(he), __FILE__, __LINE__);
 }
 
+// Packs int32 grids into the native layout.  `ninputs` grids are given;
+// replica r takes grid r / (R / ninputs) (ninputs == R: one grid per replica).
 static int engine_set_grids_impl(gasp_engine *e, const int *grids, int on_device, int ninputs) {
     const size_t bytes = (size_t)ninputs * e->N * sizeof(int);
     const int *src = grids;
@@ -1481,7 +1481,7 @@ extern "C" int gasp_engine_get_conflict_filter(gasp_engine *e, int *filter) {
 
 extern "C" int gasp_engine_get_lattice_staging(gasp_engine *e, int *staging) {
     if (!e || !staging) return set_error(GASP_ERR_ARG, "gasp_engine_get_lattice_staging: NULL argument");
-    *staging = e->win && e->method == 0 ? 3 : e->stage + 1;  // sweep_window: spins in LDS, one bit each
+    *staging = e->win && e->method == 0 ? 3 : e->stage + 1;  // sweep_window keeps the spins in LDS
     return GASP_OK;
 }
 
@@ -1594,8 +1594,8 @@ extern "C" int gasp_sweep_grids(int L, int ngrids, int gpu_method, gasp_rng_stat
 // is looked up once per device (hipGetSymbolAddress, with that device
 // current) and only that address is handed to kernels.  Calls on one device
 // share the array: calls that overlap in time on one device race.  Nothing in
-// the workspace needs to start at zero except the counters, which
-// set_thresholds clears; the lattice is written whole by the pack kernels.
+// the workspace needs to start at zero: the lattice is written whole by the
+// pack kernels, the magnetisations by the sweep.
 constexpr size_t kSweepScratchBytes = (size_t)16 << 20;
 constexpr int kScratchMaxDevices = 64;
 static __device__ __align__(256) unsigned char scratch[kSweepScratchBytes];

@@ -1533,14 +1533,6 @@ __global__ void __launch_bounds__(256) gather_spins8(const void *__restrict__ la
     }
 }
 
-// Caller grids as a sweep would leave them where none runs: any value but 1 is a
-// down spin.  (sweep_window writes no spins then; a branch for it there costs every
-// call: one sweep of 64 replicas at L = 32 15.82 us, 15.48 without.)
-__global__ void __launch_bounds__(256) only_spins(int *__restrict__ g, size_t n) {
-    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x)
-        if (g[i] != 1 && g[i] != -1) g[i] = -1;
-}
-
 __global__ void zero_ints(int *p, int n) {
     if ((int)threadIdx.x < n) p[threadIdx.x] = 0;
 }
