@@ -125,20 +125,21 @@ __device__ __forceinline__ uint32_t not_spins(uint32_t v) {
 constexpr uint32_t kNotSpins = 0x7FC51D05u;  // net_head's "pB" of a batch that is not +-1: a NaN
 
 // Spins of a group as one 64-bit mask per row (bit = column, 1 = up) to LDS;
-// absent images give zeros.  One thread per 16 columns: `it` < 4 L.
+// absent images give zeros.  One thread per 16 columns: `it` < 4 L.  True if some
+// value is not +-1.
 template <int LG>
-__device__ __forceinline__ void load_bits(const int8_t *__restrict__ s, int n, int img0, uint32_t to, int it,
-                                          int *__restrict__ odd) {
+__device__ __forceinline__ bool load_bits(const int8_t *__restrict__ s, int n, int img0, uint32_t to, int it) {
     constexpr int L = 1 << LG;
     const int row = it >> 2, col = (it & 3) * 16, img = img0 + (col >> LG);
-    uint32_t bits = 0u;
+    uint32_t bits = 0u, bad = 0u;
     if (img < n) {
         const u32x4 v = *(const u32x4 *)(s + (size_t)img * (L * L) + row * L + (col & (L - 1)));
 #pragma unroll
         for (int q = 0; q < 4; ++q) bits |= ((((~v[q] >> 7) & 0x01010101u) * 0x01020408u) >> 24 & 0xFu) << (4 * q);
-        if (not_spins(v[0]) | not_spins(v[1]) | not_spins(v[2]) | not_spins(v[3])) *odd = 1;
+        bad = not_spins(v[0]) | not_spins(v[1]) | not_spins(v[2]) | not_spins(v[3]);
     }
     lds2_set(to + 8u * (uint32_t)row + 2u * (uint32_t)(it & 3), bits);
+    return bad != 0u;
 }
 // The nine spins around (row, col) as conv1's table index (bit t = tap t).
 template <int LG>
@@ -293,7 +294,7 @@ __global__ void __launch_bounds__(kFwdThreads) net_fwd(const int8_t *__restrict_
             if (TRAIN && blockIdx.x == 0) ((uint32_t *)tab)[nine * 16 + c2] = out;
         }
     }
-    if (tid < 4 * L) load_bits<LG>(s, g.n, g.group(g.unit(0)) * kSets, kFwdBits, tid, odd);
+    if (tid < 4 * L && load_bits<LG>(s, g.n, g.group(g.unit(0)) * kSets, kFwdBits, tid)) *odd = 1;
     __syncthreads();
     // table offsets of a2 block j's six a1 rows, 4j - 3 .. 4j + 2
     auto codes = [&](const Stream &st, int buf) {
@@ -353,12 +354,17 @@ __global__ void __launch_bounds__(kFwdThreads) net_fwd(const int8_t *__restrict_
         const int lag = 2 * layer, total = K * P;
         int slot = 0;  // of block st in the layer's input ring (layers 3, 4) and in its output ring
         Stream cs;  // layer 3's waves, the least busy: conv2's block of this step
+        uint64_t bad = 0u;  // lanes that met other values than +-1 (a scalar: no vector register is left)
         for (int step = 0; step < total + 4; ++step) {
             const int i = step - lag;
             if (layer == 1 && step < total) {
                 // the next unit's spins, then the next block's table offsets
-                if (cs.j == 0 && cs.k + 1 < K && (tid & 255) < 4 * L)
-                    load_bits<LG>(s, g.n, g.group(g.unit(cs.k + 1)) * kSets, kFwdBits + (uint32_t)((cs.k + 1) & 1) * 512u, tid & 255, odd);
+                if (cs.j == 0 && cs.k + 1 < K) {
+                    bool here = false;
+                    if ((tid & 255) < 4 * L)
+                        here = load_bits<LG>(s, g.n, g.group(g.unit(cs.k + 1)) * kSets, kFwdBits + (uint32_t)((cs.k + 1) & 1) * 512u, tid & 255);
+                    bad |= __builtin_amdgcn_ballot_w64(here);
+                }
                 cs.next(P);
                 if (step + 1 < total) codes(cs, (step + 1) & 1);
             }
@@ -448,6 +454,7 @@ __global__ void __launch_bounds__(kFwdThreads) net_fwd(const int8_t *__restrict_
             }
             __syncthreads();
         }
+        if (layer == 1 && bad) *odd = 1;
     };
     if (role == 0) run(Role<0>{});
     else if (role == 1) run(Role<1>{});
