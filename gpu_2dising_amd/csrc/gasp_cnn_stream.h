@@ -17,7 +17,8 @@
 // the other, bands of four rows in chains, partials in chunks of 32), so activations,
 // gradients and trained weights are theirs bit for bit.  Inference has the same
 // activations, but pools them by eight rows (net_fwd): a grid's pB is the same bits
-// whatever the batch, and differs from the separate kernels' by float32 rounding.
+// whatever the batch (of +-1, see below), and differs from the separate kernels' by
+// float32 rounding.
 //
 // The four 16-byte chunks of a position p (64 bytes) lie in LDS at chunk ^ ((p >>
 // 2) & 3), which puts the fragment reads of 16 consecutive positions on 16
